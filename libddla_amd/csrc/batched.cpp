@@ -229,8 +229,15 @@ void pposvVbatchedTune(const DdlaHandle_t& h, char uplo, const int* d_n, T* cons
     DDLA_HIP(hipEventDestroy(e0));
     DDLA_HIP(hipEventDestroy(e1));
     DDLA_HIP(hipFree(base));
+    // The left-looking kernel rounds each element of the trailing matrix once
+    // per block column instead of once per update: on 1500 FP32 systems of
+    // orders 20 to 300 its log-determinants are 7.4e-8 off against 1.3e-7, its
+    // solutions 2.8e-7 against 4.6e-7.  So another schedule has to be faster by
+    // more than two timings of one schedule differ to be taken before it.
+    constexpr float kLeftLookingShare = 0.9f;
+    auto cost = [](const Candidate& c) { return c.left_looking ? kLeftLookingShare * c.ms : c.ms; };
     const auto best = std::min_element(cands.begin(), cands.end(),
-                                       [](const Candidate& a, const Candidate& b) { return a.ms < b.ms; });
+                                       [&](const Candidate& a, const Candidate& b) { return cost(a) < cost(b); });
     tuning = DdlaStream::BatchedTuning{true,          best->occupancy,    best->ordered,
                                        best->split_blocks, best->left_looking, best->step_blocks};
     if (occupancy) *occupancy = best->occupancy;

@@ -186,13 +186,13 @@ __device__ inline void block_apply(const T* m, long long rs, long long ks, int r
 // blocks below as L(r, j) = A(r, j) D_j^T on the matrix cores, all in place.  Returns 0, or
 // the 1-based global index of a failed pivot (then only L(j, j) is written).
 // logpart (thread 0) receives sum log L(k, k) over the block (fixed-order
-// butterfly) when with_log.  S, X: kB * kL elements of LDS each; rdiag: kB;
-// s_flag: one int.  Without the blocks below, X keeps its scratch above the
+// butterfly) when with_log.  S, X: kB * kL elements of LDS each; s_flag: one
+// int.  Without the blocks below, X keeps its scratch above the
 // diagonal (dj still gets the zeros) and no barrier follows the stores: the
 // caller synchronizes before it reads dj or reuses S and X.
 template <class T, bool OUT_OF_LINE = false>
-__device__ inline int factor_block_column(T* A, View v, int n, int nb, int j, T* dj, T* S, T* X, T* rdiag,
-                                          int* s_flag, double& logpart, bool below = true, bool with_log = true)
+__device__ inline int factor_block_column(T* A, View v, int n, int nb, int j, T* dj, T* S, T* X, int* s_flag,
+                                          double& logpart, bool below = true, bool with_log = true)
 {
     const int tid = threadIdx.x;
     const long long j0 = (long long)kB * j, lda = v.lda;
@@ -200,8 +200,8 @@ __device__ inline int factor_block_column(T* A, View v, int n, int nb, int j, T*
     T* Ajj = A + j0 + j0 * lda;
     potf2_detail::load_block<T>(v.upper != 0, wj, Ajj, lda, S);
     __syncthreads();
-    const int f = OUT_OF_LINE ? potf2_detail::factor_invert64_call<T>(S, X, rdiag, s_flag)
-                              : potf2_detail::factor_invert64<T>(S, X, rdiag, s_flag);
+    const int f = OUT_OF_LINE ? potf2_detail::factor_invert64_call<T>(S, X, s_flag)
+                              : potf2_detail::factor_invert64<T>(S, X, s_flag);
     potf2_detail::store_factor<T>(v.upper != 0, wj, S, Ajj, lda);
     if (f != 0) return (int)j0 + f;
     // log of the diagonal: wave 0, fixed-order butterfly
@@ -364,7 +364,7 @@ __device__ inline void solve_member(const T* A, View v, int n, int nb, T* Bm, lo
 template <class T, int OCC>
 __global__ __launch_bounds__(kThreads, OCC) void batched_pposv_kernel(BatchArgs<T> a)
 {
-    __shared__ T S[kB * kL], X[kB * kL], rdiag[kB];
+    __shared__ T S[kB * kL], X[kB * kL];
     __shared__ int s_item, s_flag;
     static_assert(kSlab * 4 * kB <= kB * kL && kSlab * kB <= kB * kL, "solve scratch must fit the factor buffers");
     T* const part = S;  // the solves reuse the factorization's buffers
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(kThreads, OCC) void batched_pposv_kernel(BatchArgs<
             double l = 0.0;
             // two workgroups per CU leave too few registers to inline the factorization
             const int f = factor_block_column<T, (OCC > 1)>(A, v, n, nb, j, slot + (long long)j * kB * kB, S, X,
-                                                            rdiag, &s_flag, l);
+                                                            &s_flag, l);
             if (f != 0) {
                 fail = f;
                 break;
@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256) void count_large_kernel(int batch, int max_blo
 template <class T>
 __global__ __launch_bounds__(kThreads) void blocked_panel_kernel(BlockedArgs<T> a, int j)
 {
-    __shared__ T S[kB * kL], X[kB * kL], rdiag[kB];
+    __shared__ T S[kB * kL], X[kB * kL];
     __shared__ int s_flag;
     const int b = blockIdx.x;
     if (b >= *a.count) return;
@@ -526,7 +526,7 @@ __global__ __launch_bounds__(kThreads) void blocked_panel_kernel(BlockedArgs<T> 
     }
     double lp = 0.0;
     const int f = factor_block_column<T>(a.A[item], View{lda, a.upper}, n, nb, j,
-                                         a.dinv + ((long long)b * a.max_blocks + j) * kB * kB, S, X, rdiag, &s_flag, lp,
+                                         a.dinv + ((long long)b * a.max_blocks + j) * kB * kB, S, X, &s_flag, lp,
                                          false);
     if (threadIdx.x == 0) {
         if (f != 0) a.info[item] = f;
@@ -600,13 +600,13 @@ __global__ void blocked_prep_kernel(BlockedArgs<T> a, int j, int J, StepArrays<T
 
 // LDS of the left-looking kernel, in elements of T: the larger of the
 // products' double-buffered slabs (128 x 64 tiles), the diagonal block's S,
-// X and rdiag, and the solve's kLLCols-column right-hand-side buffer.
+// X, and the solve's kLLCols-column right-hand-side buffer.
 constexpr int kLLCols = 4;
 template <class T>
 constexpr int ll_lds_elems()
 {
     constexpr int g = gemm_detail::lds_elems<128, 64, 16>();
-    constexpr int f = 2 * kB * kL + kB;
+    constexpr int f = 2 * kB * kL;
     constexpr int s = kMaxBlocks * kB * kLLCols;
     return g > f ? (g > s ? g : s) : (f > s ? f : s);
 }
@@ -809,9 +809,8 @@ __device__ inline int ll_block_column(T* A, View v, int n, int nb, int j, T* dj,
     }
     T* S = smem;
     T* X = smem + kB * kL;
-    T* rdiag = smem + 2 * kB * kL;
     double unused = 0.0;
-    const int f = factor_block_column<T, (OCC > 1)>(A, v, n, nb, j, dj, S, X, rdiag, s_flag, unused, false, false);
+    const int f = factor_block_column<T, (OCC > 1)>(A, v, n, nb, j, dj, S, X, s_flag, unused, false, false);
     if (f != 0) return f;
     __syncthreads();
     if (m > kB) {

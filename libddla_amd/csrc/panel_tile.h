@@ -180,7 +180,7 @@ struct Acc64 {
 template <class T>
 __global__ __launch_bounds__(256) void panel_kernel(PanelArgs<T> a)
 {
-    __shared__ T S[kB * kL], X[kB * kL], rdiag[kB];
+    __shared__ T S[kB * kL], X[kB * kL];
     __shared__ int s_ticket, s_flag;
     const int tid = threadIdx.x;
     if (gridDim.y > 1) {
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void panel_kernel(PanelArgs<T> a)
     __syncthreads();
     if (tid >= h && tid < kB) S[tid * kL + tid] = T(1);
     __syncthreads();
-    const int fail = potf2_detail::factor_invert64<T>(S, X, rdiag, &s_flag);
+    const int fail = potf2_detail::factor_invert64<T>(S, X, &s_flag);
     potf2_detail::store_factor<T>(a.upper != 0, h, S, a.A + r0 + r0 * a.lda, a.lda);
     if (fail != 0) {
         if (tid == 0) {
