@@ -35,19 +35,29 @@ constexpr int kIB = 64;  // diagonal block of potf2 and of the solves
 // Outer panel width of the factorization: the depth of the trailing-update
 // GEMM.  Not the descriptor's NB -- at 1 x 1 the block size of the
 // distribution does not change the arithmetic (the reference hands the whole
-// matrix to one ?potrf call).  Deeper updates amortize each tile's C
-// read-modify-write better, wider panels lengthen the panel chain: FP64 at
-// n = 32768 ran 209.3 / 205.0 / 206.4 ms with 512 / 768 / 1024, while at
-// n = 4096 (panel-bound) 512 is best.  The split-product path keeps 512 (its
-// panel buffers hold 512 columns).
+// matrix to one ?potrf call).
+// * A single problem of order <= 4096 is one panel: its 64 x 64 blocks are units
+//   of one launch, whose chain of diagonal blocks (18 us each in FP64) is all
+//   that is left; by 512-column panels the chain also waits for the rows below
+//   each panel, the look-ahead update of the next and two stream hand-overs:
+//   n = 2048 took 1.0 ms then, 0.6 ms now.
+// * Beyond, deeper updates amortize each tile's C read-modify-write better, wider
+//   panels lengthen the panel chain: FP64 at n = 32768 ran 209.3 / 205.0 / 206.4
+//   ms with 512 / 768 / 1024, while at n = 8192 512 is best.
+// * A batch of problems fills the chip with 512-column panels, which leave more
+//   of the work to the trailing updates; the split-product path keeps 512 (its
+//   panel buffers hold 512 columns).  With the launch profiler on, whose classes
+//   are the steps of the panel schedule, small orders take 512 too.
 // A process-wide override (set_panel_width; 0 = the rule above) lets tests
-// run the 768-column panels at small orders.
+// run narrower and the 768-column panels at small orders.
 std::atomic<int> g_panel_width{0};
+constexpr int kOnePanelOrder = 4096;
 template <class T>
-int outer_block(int n, bool split)
+int outer_block(int n, bool split, bool one_panel = true)
 {
     const int w = g_panel_width.load(std::memory_order_relaxed);
     if (w > 0) return split ? std::min(w, 512) : w;
+    if (!split && one_panel && n <= kOnePanelOrder) return kOnePanelOrder;
     return std::is_same<T, double>::value && n >= 16384 ? 768 : 512;
 }
 
@@ -85,7 +95,7 @@ void factor_panel(DdlaStream* h, hipStream_t st, const LView<T>& v, int n, int k
 {
     const double below = (double)n - k - kb;
     LaunchTimer timer(h, kClassPanel, ((double)kb * kb * kb / 3.0 + below * kb * kb) * batch.count, 0, st);
-    kern::panel_factor<T>(st, false, n, v.A, v.lda, k, kb, info, work, batch);
+    kern::panel_factor<T>(st, n, v.A, v.lda, k, kb, info, work, batch);
 }
 
 // Split-product trailing updates (FP32 factorization only): after panel p is
@@ -223,7 +233,7 @@ void potrf_blocked(DdlaStream* h, bool upper, int n, T* A, long long lda, int* i
         return;
     }
     const LView<T> v{A, lda};
-    const int NB = outer_block<T>(n, split != nullptr);
+    const int NB = outer_block<T>(n, split != nullptr, batch.count == 1 && !h->profiling);
     const int np = (n + NB - 1) / NB;
     hipStream_t main = h->stream, side = h->side, look = h->look;
     auto col = [&](int q) { return std::min(n, q * NB); };  // first column of panel q (n past the end)

@@ -67,10 +67,9 @@ void vbatched_validate(hipStream_t s, int na, int nb, const int* m, const int* n
                        const int* ldb, const int* ldc, int batch, int* summary);
 
 // Panel factorization of the blocked Cholesky (one persistent launch per
-// panel).  The factor is addressed as an "L view": element (i, j), i >= j, at
-// A[i + j*lda], or A[j + i*lda] when upper.  panel_factor factors columns
-// [k, k + kb) (kb <= 768, every earlier trailing update applied): the
-// diagonal blocks, their inverses and the rows below.  On a non-positive or
+// panel), T real or std::complex.  panel_factor factors columns [k, k + kb) (kb
+// <= 4096, every earlier trailing update applied) of the lower triangle at A:
+// the diagonal blocks, their inverses and the rows below.  On a non-positive or
 // NaN pivot in global column p (0-based) it sets *info = p + 1, and
 // kInfoWaitLimit if one of its waits gave up (unless *info was set first); it
 // does nothing if *info != 0 on entry.  work holds panel_work_bytes<T>(n) bytes,
@@ -84,11 +83,11 @@ void panel_reset(hipStream_t s, int n, void* work, const Batch& batch = Batch())
 template <class T>
 int* panel_error_word(int n, void* work);
 template <class T>
-void panel_factor(hipStream_t s, bool upper, int n, T* A, long long lda, int k, int kb, int* info, void* work,
+void panel_factor(hipStream_t s, int n, T* A, long long lda, int k, int kb, int* info, void* work,
                   const Batch& batch = Batch());
 
-// Split-product trailing update of the FP32 factorization (L view as for
-// panel_factor); mode = 1 (bf16x3: two bfloat16 planes, three products), 2
+// Split-product trailing update of the FP32 factorization (L view: element (i,
+// j), i >= j, of the factor at A[i + j*lda], or A[j + i*lda] when upper); mode = 1 (bf16x3: two bfloat16 planes, three products), 2
 // (bf16x6: three planes, six products) or 3 (fp16x3: two half-precision
 // planes of row-scaled values, three products).  split_panel writes rows
 // [0, m) and columns [0, kb) (kb <= 512) of the L view starting at X -- the
@@ -108,7 +107,7 @@ void split_update(hipStream_t s, int mode, bool upper, int m, int n2, int kb, co
                   int a_row, int b_row, float* C, long long ldc, bool tri, long long diag, const int* abort);
 
 // Inverts every 64 x 64 diagonal block of the order-n factor (L view as for
-// panel_factor) into inv[b * 4096 ...], identity-padded for a ragged last
+// split_update) into inv[b * 4096 ...], identity-padded for a ragged last
 // block; unit: the diagonal is taken as ones (the stored one is not used).
 template <class T>
 void trtri_diag_blocks(hipStream_t s, bool upper, int n, const T* A, long long lda, T* inv, bool unit = false,
@@ -119,7 +118,7 @@ template <class T>
 void scale_matrix(hipStream_t s, int m, int n, T alpha, T* M, long long ld);
 
 // Forward (L Y = B) then backward (L^T X = Y) substitution with the order-n
-// factor (L view as for panel_factor) and its inverted 64 x 64 diagonal blocks
+// factor (L view as for split_update) and its inverted 64 x 64 diagonal blocks
 // dinv (from trtri_diag_blocks), in place on B (n x nrhs), one launch per
 // sweep.  work must hold solve_work_bytes(nrhs) bytes; *error (device) is set
 // to 1 if a sweep's internal wait ever exceeded its limit (the result is then

@@ -10,6 +10,7 @@
 #include "solve_tile.h"
 #include "stage_tile.h"
 #include "potf2_tile.h"
+#include "panel_host.h"
 #include "panel_tile.h"
 #include "batched_tile.h"
 #include "split_tile.h"
@@ -650,71 +651,6 @@ void vbatched_validate(hipStream_t s, int na, int nb, const int* m, const int* n
 {
     vbatched_validate_kernel<<<1, 256, 0, s>>>(na, nb, m, n, k, lda, ldb, ldc, batch, summary);
     check_launch("vbatched_validate");
-}
-
-// panel work: [ kMaxCols inverses | kSyncInts counters per 64-column block | error word ]
-template <class T>
-size_t panel_work_bytes(int n)
-{
-    using namespace panel_detail;
-    const size_t nb = (size_t)(n + kB - 1) / kB;
-    return ((size_t)kMaxCols * kB * kB * sizeof(T) + 255) / 256 * 256 + ((nb * kSyncInts + 1) * sizeof(int) + 255) / 256 * 256;
-}
-
-namespace {
-template <class T>
-int* panel_sync(void* work)
-{
-    using namespace panel_detail;
-    return reinterpret_cast<int*>(static_cast<char*>(work) + ((size_t)kMaxCols * kB * kB * sizeof(T) + 255) / 256 * 256);
-}
-} // namespace
-
-template <class T>
-int* panel_error_word(int n, void* work)
-{
-    using namespace panel_detail;
-    return panel_sync<T>(work) + (size_t)((n + kB - 1) / kB) * kSyncInts;
-}
-
-namespace {
-// p[0, count) := 0 for each problem y (problem y's words stride bytes after problem 0's)
-__global__ void zero_ints_batched_kernel(int* p, int count, long long stride)
-{
-    int* q = reinterpret_cast<int*>(reinterpret_cast<char*>(p) + blockIdx.y * stride);
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) q[i] = 0;
-}
-} // namespace
-
-template <class T>
-void panel_reset(hipStream_t s, int n, void* work, const Batch& batch)
-{
-    using namespace panel_detail;
-    const int count = ((n + kB - 1) / kB) * kSyncInts + 1;
-    if (batch.count == 1) {
-        solve_detail::zero_ints_kernel<<<grid_for(count, 256), 256, 0, s>>>(panel_sync<T>(work), count);
-    } else if (batch.count > 1) {
-        const dim3 grid((unsigned)grid_for(count, 256), (unsigned)batch.count);
-        zero_ints_batched_kernel<<<grid, 256, 0, s>>>(panel_sync<T>(work), count, batch.stride);
-    }
-    check_launch("panel_reset");
-}
-
-template <class T>
-void panel_factor(hipStream_t s, bool upper, int n, T* A, long long lda, int k, int kb, int* info, void* work,
-                  const Batch& batch)
-{
-    using namespace panel_detail;
-    if (kb <= 0 || k < 0 || k + kb > n) return;
-    if (kb > kMaxCols * kB) throw std::invalid_argument("panel_factor: panel wider than 768 columns");
-    if (k % kB != 0) throw std::invalid_argument("panel_factor: panel must start on a 64-column boundary");
-    PanelArgs<T> a{A, lda, upper ? 1 : 0, n, k, kb, info, static_cast<T*>(work),
-                   panel_sync<T>(work) + (size_t)(k / kB) * kSyncInts, panel_error_word<T>(n, work), wait_limit(),
-                   batch.stride};
-    const int rows = (n - k + kB - 1) / kB;
-    if (batch.count <= 0) return;
-    panel_kernel<T><<<dim3((unsigned)rows, (unsigned)batch.count), 256, 0, s>>>(a);
-    check_launch("panel_factor");
 }
 
 template <class T>
@@ -1368,7 +1304,7 @@ void convert(hipStream_t s, int m, int n, const S* in, long long ldi, D* out, lo
     template size_t panel_work_bytes<T>(int);                                                                 \
     template void panel_reset<T>(hipStream_t, int, void*, const Batch&);                                      \
     template int* panel_error_word<T>(int, void*);                                                            \
-    template void panel_factor<T>(hipStream_t, bool, int, T*, long long, int, int, int*, void*, const Batch&); \
+    template void panel_factor<T>(hipStream_t, int, T*, long long, int, int, int*, void*, const Batch&);       \
     template void batched_pposv<T>(hipStream_t, bool, int, int, const int*, T* const*, const int*, T* const*,  \
                                    const int*, int*, double*, int, int, bool, int, int, void*, bool, int);     \
     template void batched_copy<T>(hipStream_t, int, const int*, int, T* const*, const int*, T* const*,         \

@@ -1,9 +1,11 @@
 // Cholesky factorization and triangular inverse of one 64 x 64 diagonal block
 // held in LDS, for a 256-thread workgroup on gfx950 (device code, included by
-// kernels.hip).
+// kernels.hip and zkernels.hip), real or complex Hermitian.
 //
 // The block S is column-major in LDS with column stride kL (S[c * kL + r] =
-// A(r, c)) and only its lower triangle is referenced.  It is factored in
+// A(r, c); of a complex block the real parts, kPlane elements before the
+// imaginary ones) and only its lower triangle is referenced, of its diagonal
+// only the real part.  It is factored in
 // 16-column strips, the inverse X = L^-1 growing beside it:
 //   * a strip is factored four columns at a time on the matrix cores
 //     (factor_strip).  Every wavefront keeps the strip's 16 x 16 diagonal
@@ -28,6 +30,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "field.h"
 #include "gemm_tile.h"
 
 namespace ddla {
@@ -35,17 +38,38 @@ namespace kern {
 namespace potf2_detail {
 
 using gemm_detail::Mfma;
+using namespace field;
 
-constexpr int kB = 64;  // block order
-constexpr int kL = 65;  // LDS column stride, in elements
-constexpr int kW = 16;  // strip width
+constexpr int kB = 64;           // block order
+constexpr int kL = 65;           // LDS column stride, in elements
+constexpr int kPlane = kB * kL;  // one plane of a block in LDS
+constexpr int kW = 16;           // strip width
+
+// A wavefront's accumulators of one 16 x 16 tile of T.
+template <class T>
+using tile_acc = acc_t<real_t<T>>[Field<T>::planes];
+
+template <class T>
+__device__ __forceinline__ void clear(tile_acc<T>& acc)
+{
+#pragma unroll
+    for (int p = 0; p < Field<T>::planes; ++p) acc[p] = acc_t<real_t<T>>{0, 0, 0, 0};
+}
+
+// Element idx of a block in LDS, of every plane.
+template <class T>
+__device__ __forceinline__ void load_planes(const real_t<T>* S, real_t<T> (&v)[Field<T>::planes])
+{
+#pragma unroll
+    for (int p = 0; p < Field<T>::planes; ++p) v[p] = S[p * kPlane];
+}
 
 template <int i>
 struct Const {
     static constexpr int value = i;
 };
 
-__device__ inline double lane_value(double x, int l)
+__device__ __forceinline__ double lane_value(double x, int l)
 {
     const long long b = __double_as_longlong(x);
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
@@ -53,40 +77,40 @@ __device__ inline double lane_value(double x, int l)
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-__device__ inline float lane_value(float x, int l)
+__device__ __forceinline__ float lane_value(float x, int l)
 {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
 }
 
 // x where mask is all ones, zero where it is zero (whatever x is).
-__device__ inline double masked(double x, int mask)
+__device__ __forceinline__ double masked(double x, int mask)
 {
     const long long b = __double_as_longlong(x);
     const unsigned lo = (unsigned)b & (unsigned)mask, hi = (unsigned)(b >> 32) & (unsigned)mask;
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-__device__ inline float masked(float x, int mask) { return __int_as_float(__float_as_int(x) & mask); }
+__device__ __forceinline__ float masked(float x, int mask) { return __int_as_float(__float_as_int(x) & mask); }
 
 // The bits of x and y together (one of them masked to zero).
-__device__ inline double merged(double x, double y)
+__device__ __forceinline__ double merged(double x, double y)
 {
     return __longlong_as_double(__double_as_longlong(x) | __double_as_longlong(y));
 }
 
-__device__ inline float merged(float x, float y) { return __int_as_float(__float_as_int(x) | __float_as_int(y)); }
+__device__ __forceinline__ float merged(float x, float y) { return __int_as_float(__float_as_int(x) | __float_as_int(y)); }
 
 // 1 / sqrt(d) for d > 0: the hardware estimate and one third-order step (FP64:
 // with e = 1 - d y^2, y (1 + e/2 + 3 e^2 / 8); the estimate's ~2^-23 becomes
 // ~2^-67, rounding aside) or one Newton step (FP32).
-__device__ inline double rsqrt_refined(double d)
+__device__ __forceinline__ double rsqrt_refined(double d)
 {
     const double y = __builtin_amdgcn_rsq(d);
     const double e = fma(-(d * y), y, 1.0);
     return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-__device__ inline float rsqrt_refined(float d)
+__device__ __forceinline__ float rsqrt_refined(float d)
 {
     float y = __builtin_amdgcn_rsqf(d);
     const float h = 0.5f * d;
@@ -99,10 +123,10 @@ __device__ inline float rsqrt_refined(float d)
 // columns 4q .. 4q + 3 (column 4q + lane / 16) and can serve as the product's
 // left operand too.  FP64 accumulators are D[l / 16 + 4r][l % 16], FP32 ones
 // D[4 (l / 16) + r][l % 16].
-template <class T>
+template <class R>
 __device__ constexpr int diag_row(int i)
 {
-    return sizeof(T) == 8 ? i : (i >> 2) + 4 * (i & 3);  // its own inverse
+    return sizeof(R) == 8 ? i : (i >> 2) + 4 * (i & 3);  // its own inverse
 }
 
 // One wavefront's share of strip b (columns 16b .. 16b+15): wavefront w < 4 - b
@@ -115,230 +139,259 @@ __device__ constexpr int diag_row(int i)
 // meaningful values.  No branch depends on a pivot (a failed one is recorded,
 // not acted on).
 template <class T, int b>
-__device__ __attribute__((always_inline)) inline int factor_strip(T* S, T* X, T (&diag)[4])
+__device__ __forceinline__ int factor_strip(real_t<T>* S, real_t<T>* X,
+                                                                  real_t<T> (&diag)[4][Field<T>::planes])
 {
-    using Op = Mfma<T>;
-    using acc_t = typename Op::acc_t;
+    using R = real_t<T>;
+    constexpr int P = Field<T>::planes;
     constexpr int r0 = kW * b;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
-    const int pr = diag_row<T>(li);
-    acc_t d, x;
+    const int pr = diag_row<R>(li);
+    tile_acc<T> d, x;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int c = g + 4 * r;
-        d[r] = masked(S[(r0 + c) * kL + r0 + pr], -(int)(pr >= c));
-        x[r] = wave == 0 ? (li == c ? T(1) : T(0)) : S[(r0 + c) * kL + r0 + kW * wave + li];
-    }
-    const T u0 = g == 0 ? T(1) : T(0), u1 = g == 1 ? T(1) : T(0), u2 = g == 2 ? T(1) : T(0), u3 = g == 3 ? T(1) : T(0);
-    T below[4];                  // the finished columns of x
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = g + 4 * r;
+            d[p][r] = masked(S[p * kPlane + (r0 + c) * kL + r0 + pr], -(int)(p == 0 ? pr >= c : pr > c));
+            x[p][r] = wave == 0 ? (p == 0 && li == c ? R(1) : R(0))
+                                : S[p * kPlane + (r0 + c) * kL + r0 + kW * wave + li];
+        }
+    auto unit = [&](int k) { return element<T>(g == k ? R(1) : R(0), R(0)); };
+    const T u1 = unit(1), u2 = unit(2), u3 = unit(3);
+    R below[4][P];               // the finished columns of x
     unsigned long long bad = 0;  // bit j: the pivot of column j is not positive
-    auto check = [&](T p, int j) { bad |= __ballot(!(p > T(0))) & (1ull << j); };
+    auto check = [&](R v, int j) { bad |= __ballot(!(v > R(0))) & (1ull << j); };
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        auto at = [&](int r, int c) { return lane_value(d[q], 16 * c + diag_row<T>(4 * q + r)); };
-        const T a00 = at(0, 0), a10 = at(1, 0), a20 = at(2, 0), a30 = at(3, 0), a11 = at(1, 1);
-        const T a21 = at(2, 1), a31 = at(3, 1), a22 = at(2, 2), a32 = at(3, 2), a33 = at(3, 3);
-        const T y0 = rsqrt_refined(a00);
-        const T l10 = a10 * y0, l20 = a20 * y0, l30 = a30 * y0;
-        const T d1 = fma(-l10, l10, a11), y1 = rsqrt_refined(d1);
-        const T l21 = fma(-l20, l10, a21) * y1, l31 = fma(-l30, l10, a31) * y1;
-        const T d2 = fma(-l21, l21, fma(-l20, l20, a22)), y2 = rsqrt_refined(d2);
-        const T l32 = fma(-l31, l21, fma(-l30, l20, a32)) * y2;
-        const T d3 = fma(-l32, l32, fma(-l31, l31, fma(-l30, l30, a33))), y3 = rsqrt_refined(d3);
+        auto real_at = [&](int c) { return lane_value(d[0][q], 16 * c + diag_row<R>(4 * q + c)); };
+        auto at = [&](int r, int c) {
+            const int l = 16 * c + diag_row<R>(4 * q + r);
+            return element<T>(lane_value(d[0][q], l), lane_value(d[P - 1][q], l));
+        };
+        const R a00 = real_at(0), a11 = real_at(1), a22 = real_at(2), a33 = real_at(3);
+        const T a10 = at(1, 0), a20 = at(2, 0), a30 = at(3, 0), a21 = at(2, 1), a31 = at(3, 1), a32 = at(3, 2);
+        const R y0 = rsqrt_refined(a00);
+        const T l10 = scale(a10, y0), l20 = scale(a20, y0), l30 = scale(a30, y0);
+        const R d1 = sub_norm(a11, l10), y1 = rsqrt_refined(d1);
+        const T l21 = scale(sub_mul_conj(a21, l20, l10), y1), l31 = scale(sub_mul_conj(a31, l30, l10), y1);
+        const R d2 = sub_norm(sub_norm(a22, l20), l21), y2 = rsqrt_refined(d2);
+        const T l32 = scale(sub_mul_conj(sub_mul_conj(a32, l30, l20), l31, l21), y2);
+        const R d3 = sub_norm(sub_norm(sub_norm(a33, l30), l31), l32), y3 = rsqrt_refined(d3);
         check(a00, 4 * q);
         check(d1, 4 * q + 1);
         check(d2, 4 * q + 2);
         check(d3, 4 * q + 3);
         // column g of the 4 x 4 inverse, then its row diag_row(l % 16) as the left operand
-        const T e0 = u0 * y0, e1 = fma(-l10, e0, u1) * y1;
-        const T e2 = fma(-l21, e1, fma(-l20, e0, u2)) * y2;
-        const T e3 = fma(-l32, e2, fma(-l31, e1, fma(-l30, e0, u3))) * y3;
-        const T inv = merged(merged(masked(e0, -(int)(pr == 0)), masked(e1, -(int)(pr == 1))),
-                             merged(masked(e2, -(int)(pr == 2)), masked(e3, -(int)(pr == 3))));
-        const acc_t zero = {0, 0, 0, 0};
-        diag[q] = Op::mma(inv, d[q], zero)[0];
-        if (q < 3) d = Op::mma(masked(-diag[q], -(int)(pr >= 4 * q + 4)), diag[q], d);
-        below[q] = Op::mma(inv, x[q], zero)[0];
-        if (q < 3) x = Op::mma(masked(-diag[q], -(int)(pr >= 4 * q + 4)), below[q], x);
+        const T e0 = scale(unit(0), y0), e1 = scale(sub_mul(u1, l10, e0), y1);
+        const T e2 = scale(sub_mul(sub_mul(u2, l20, e0), l21, e1), y2);
+        const T e3 = scale(sub_mul(sub_mul(sub_mul(u3, l30, e0), l31, e1), l32, e2), y3);
+        R inv[P], next[P], own[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            inv[p] = merged(merged(masked(plane(e0, p), -(int)(pr == 0)), masked(plane(e1, p), -(int)(pr == 1))),
+                            merged(masked(plane(e2, p), -(int)(pr == 2)), masked(plane(e3, p), -(int)(pr == 3))));
+            own[p] = d[p][q];
+        }
+        // the four finished columns W = A L44^-H, transposed: conj(inv) times the register
+        tile_acc<T> w;
+        clear<T>(w);
+        mma_conj_add(inv, own, w);
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            diag[q][p] = w[p][0];
+            next[p] = masked(-w[p][0], -(int)(pr >= 4 * q + 4));  // the rows that later columns multiply
+        }
+        if (q < 3) mma_conj_add(next, diag[q], d);
+#pragma unroll
+        for (int p = 0; p < P; ++p) own[p] = x[p][q];
+        clear<T>(w);
+        mma_conj_add(inv, own, w);
+#pragma unroll
+        for (int p = 0; p < P; ++p) below[q][p] = w[p][0];
+        if (q < 3) mma_conj_add(next, below[q], x);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int c = g + 4 * r;
-        if (wave == 0) X[(r0 + li) * kL + r0 + c] = below[r];
-        else S[(r0 + c) * kL + r0 + kW * wave + li] = below[r];
-    }
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = g + 4 * r;
+            if (wave == 0) X[p * kPlane + (r0 + li) * kL + r0 + c] = p == 0 ? below[r][p] : -below[r][p];
+            else S[p * kPlane + (r0 + c) * kL + r0 + kW * wave + li] = below[r][p];
+        }
     return bad == 0 ? 0 : r0 + (int)__ffsll(bad);
 }
 
 // L(b, b), as factor_strip left it in a wavefront's diag, to S.
 template <class T>
-__device__ __attribute__((always_inline)) inline void store_diagonal(const T (&diag)[4], int b, T* S)
+__device__ __forceinline__ void store_diagonal(const real_t<T> (&diag)[4][Field<T>::planes],
+                                                                     int b, real_t<T>* S)
 {
-    const int lane = threadIdx.x & 63, pr = diag_row<T>(lane & 15);
+    const int lane = threadIdx.x & 63, pr = diag_row<real_t<T>>(lane & 15);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int c = (lane >> 4) + 4 * r;
-        if (pr >= c) S[(kW * b + c) * kL + kW * b + pr] = diag[r];
-    }
+    for (int p = 0; p < Field<T>::planes; ++p)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = (lane >> 4) + 4 * r;
+            if (pr >= c)
+                S[p * kPlane + (kW * b + c) * kL + kW * b + pr] = p == 1 && pr == c ? real_t<T>(0) : diag[r][p];
+        }
 }
 
-// S(16r.., 16c..) -= L(16r.., strip b) L(16c.., strip b)^T, one 16 x 16 tile by
+// S(16r.., 16c..) -= L(16r.., strip b) L(16c.., strip b)^H, one 16 x 16 tile by
 // one wavefront.
 template <class T>
-__device__ __attribute__((always_inline)) inline void update_tile(T* S, int b, int r, int c)
+__device__ __forceinline__ void update_tile(real_t<T>* S, int b, int r, int c)
 {
-    using Op = Mfma<T>;
+    using R = real_t<T>;
+    using Op = Mfma<R>;
+    constexpr int P = Field<T>::planes;
     const int lane = threadIdx.x & 63, li = lane & 15;
-    T* C = S + (kW * c + li) * kL + kW * r;
-    typename Op::acc_t acc;
+    R* C = S + (kW * c + li) * kL + kW * r;
+    tile_acc<T> acc;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] = C[Op::row(lane, e)];
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[p][e] = C[p * kPlane + Op::row(lane, e)];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const T* k = S + (kW * b + Op::row(lane, s)) * kL + li;
-        acc = Op::mma(-k[kW * r], k[kW * c], acc);
+        const R* k = S + (kW * b + Op::row(lane, s)) * kL + li;
+        R left[P], right[P];
+        load_planes<T>(k + kW * r, left);
+        load_planes<T>(k + kW * c, right);
+        mma_sub_conj(left, right, acc);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) C[Op::row(lane, e)] = acc[e];
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) C[p * kPlane + Op::row(lane, e)] = acc[p][e];
 }
 
-// acc + A B of two 16 x 16 tiles given by their first elements.  The product
+// acc += A B of two 16 x 16 tiles given by their first elements.  The product
 // steps take the inner index in the order of the accumulator's rows
 // (Op::row(lane, s) in step s), so that an accumulator can be the right
 // operand of a following product as it stands (left_product).
 template <class T>
-__device__ __attribute__((always_inline)) inline typename Mfma<T>::acc_t tile_product(
-    const T* A, const T* B, typename Mfma<T>::acc_t acc)
+__device__ __forceinline__ void tile_product(const real_t<T>* A, const real_t<T>* B,
+                                                                   tile_acc<T>& acc)
 {
-    using Op = Mfma<T>;
+    using R = real_t<T>;
+    constexpr int P = Field<T>::planes;
     const int lane = threadIdx.x & 63, li = lane & 15;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const int k = Op::row(lane, s);
-        acc = Op::mma(A[k * kL + li], B[li * kL + k], acc);
+        const int k = Mfma<R>::row(lane, s);
+        R left[P], right[P];
+        load_planes<T>(A + k * kL + li, left);
+        load_planes<T>(B + li * kL + k, right);
+        mma_add(left, right, acc);
     }
-    return acc;
 }
 
 // C = -D t: D and C 16 x 16 tiles in LDS, t an accumulator.
 template <class T>
-__device__ __attribute__((always_inline)) inline void left_product(const T* D, const typename Mfma<T>::acc_t& t, T* C)
+__device__ __forceinline__ void left_product(const real_t<T>* D, const tile_acc<T>& t,
+                                                                   real_t<T>* C)
 {
-    using Op = Mfma<T>;
+    using R = real_t<T>;
+    using Op = Mfma<R>;
+    constexpr int P = Field<T>::planes;
     const int lane = threadIdx.x & 63, li = lane & 15;
-    typename Op::acc_t acc = {0, 0, 0, 0};
+    tile_acc<T> acc;
+    clear<T>(acc);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) acc = Op::mma(-D[Op::row(lane, s) * kL + li], t[s], acc);
+    for (int s = 0; s < 4; ++s) {
+        R left[P], right[P];
+        load_planes<T>(D + Op::row(lane, s) * kL + li, left);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) C[li * kL + Op::row(lane, e)] = acc[e];
+        for (int p = 0; p < P; ++p) {
+            left[p] = -left[p];
+            right[p] = t[p][s];
+        }
+        mma_add(left, right, acc);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) C[p * kPlane + li * kL + Op::row(lane, e)] = acc[p][e];
 }
 
-// X = L^-1 for the lower triangle of S, rdiag[i] = 1 / L(i, i).  The lower
-// triangle of X is complete on return; its strict upper triangle holds
-// scratch (callers write zeros there when they store X).
+// X = L^-1 for the lower triangle of S, rdiag[i] = 1 / L(i, i) (real).  The
+// lower triangle of X is complete on return, with zeros above the diagonal in
+// its diagonal 16 x 16 blocks; the blocks above those are not written.
 template <class T>
-__device__ __attribute__((always_inline)) inline void invert_lower(const T* S, const T* rdiag, T* X)
+__device__ __forceinline__ void invert_lower(const real_t<T>* S, const real_t<T>* rdiag,
+                                                                   real_t<T>* X)
 {
-    using Op = Mfma<T>;
-    using acc_t = typename Op::acc_t;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    using R = real_t<T>;
+    constexpr int P = Field<T>::planes;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    auto s_at = [&](int r, int c) { return S + kW * c * kL + kW * r; };
+    auto x_at = [&](int r, int c) { return X + kW * c * kL + kW * r; };
     // diagonal 16 x 16 inverses; in wavefront p, lane c < 16 owns column c of D(p)
     {
         const int o = kW * wave;
         T x[kW];
 #pragma unroll
         for (int i = 0; i < kW; ++i) {
-            T t = (i == lane) ? T(1) : T(0);
+            T t = element<T>(i == lane ? R(1) : R(0), R(0));
 #pragma unroll
-            for (int k = 0; k < i; ++k) t = fma(-S[(o + k) * kL + o + i], x[k], t);
-            x[i] = t * rdiag[o + i];
+            for (int k = 0; k < i; ++k) {
+                R l[P];
+                load_planes<T>(S + (o + k) * kL + o + i, l);
+                t = sub_mul(t, element<T>(l[0], l[P - 1]), x[k]);
+            }
+            x[i] = scale(t, rdiag[o + i]);
         }
         if (lane < kW) {
 #pragma unroll
-            for (int i = 0; i < kW; ++i) X[(o + lane) * kL + o + i] = x[i];
+            for (int i = 0; i < kW; ++i)
+#pragma unroll
+                for (int p = 0; p < P; ++p) X[p * kPlane + (o + lane) * kL + o + i] = plane(x[i], p);
         }
     }
     __syncthreads();
-    // X(r, c) = -D(r) L(r, c) D(c) for (r, c) = (1, 0), (3, 2); T = L(r, c) D(c)
-    // is staged in the unused block X(c, r)
-    const int r2 = 2 * wave + 1, c2 = 2 * wave;
-    if (wave < 2) {
-        acc_t acc = {0, 0, 0, 0};
+    // X(r, c) = -D(r) sum_{c <= k < r} L(r, k) X(k, c), one subdiagonal of blocks at a time
 #pragma unroll
-        for (int ks = 0; ks < kW; ks += 4) {
-            const int kk = ks + lk;
-            acc = Op::mma(S[(kW * c2 + kk) * kL + kW * r2 + li], X[(kW * c2 + li) * kL + kW * c2 + kk], acc);
+    for (int s = 1; s < 4; ++s) {
+        if (wave + s < 4) {
+            tile_acc<T> t;
+            clear<T>(t);
+            for (int k = wave; k < wave + s; ++k) tile_product<T>(s_at(wave + s, k), x_at(k, wave), t);
+            left_product<T>(x_at(wave + s, wave + s), t, x_at(wave + s, wave));
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) X[(kW * r2 + li) * kL + kW * c2 + Op::row(lane, e)] = acc[e];
+        __syncthreads();
     }
-    __syncthreads();
-    if (wave < 2) {
-        acc_t acc = {0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < kW; ks += 4) {
-            const int kk = ks + lk;
-            acc = Op::mma(-X[(kW * r2 + kk) * kL + kW * r2 + li], X[(kW * r2 + li) * kL + kW * c2 + kk], acc);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) X[(kW * c2 + li) * kL + kW * r2 + Op::row(lane, e)] = acc[e];
-    }
-    __syncthreads();
-    // X21 = -X22 (L21 X11) on 32-row halves; wavefront w owns 16 x 16 tile
-    // (a, bc) = (w / 2, w % 2); T = L21 X11 is staged in the unused X[0:32, 32:64]
-    const int a = wave >> 1, bc = wave & 1;
-    {
-        acc_t acc = {0, 0, 0, 0};
-        for (int kb = bc; kb < 2; ++kb) {
-#pragma unroll
-            for (int ks = 0; ks < kW; ks += 4) {
-                const int kk = kW * kb + ks + lk;
-                acc = Op::mma(S[kk * kL + 32 + kW * a + li], X[(kW * bc + li) * kL + kk], acc);
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) X[(32 + kW * bc + li) * kL + kW * a + Op::row(lane, e)] = acc[e];
-    }
-    __syncthreads();
-    {
-        acc_t acc = {0, 0, 0, 0};
-        for (int kb = 0; kb <= a; ++kb) {
-#pragma unroll
-            for (int ks = 0; ks < kW; ks += 4) {
-                const int kk = kW * kb + ks + lk;
-                acc = Op::mma(-X[(32 + kk) * kL + 32 + kW * a + li], X[(32 + kW * bc + li) * kL + kk], acc);
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) X[(kW * bc + li) * kL + 32 + kW * a + Op::row(lane, e)] = acc[e];
-    }
-    __syncthreads();
 }
 
 // Factorization of the lower triangle of S in place and, when it succeeds,
 // X = L^-1 (its lower triangle; the 16 x 16 blocks above the diagonal are not
 // written).  Returns 0 or the 1-based index of the first failed pivot (uniform
 // over the workgroup).  Every thread of the workgroup must call it, and it
-// ends with a barrier.
-template <class T>
-__device__ __attribute__((always_inline)) inline int factor_invert64(T* S, T* X, int* s_flag)
+// ends with a barrier.  before() and after() run on every thread around the
+// barrier that ends the first strip.
+template <class T, class Before, class After>
+__device__ __forceinline__ int factor_invert64(real_t<T>* S, real_t<T>* X, int* s_flag,
+                                                                     Before before, After after)
 {
     const int wave = threadIdx.x >> 6;
     auto s_at = [&](int r, int c) { return S + kW * c * kL + kW * r; };
     auto x_at = [&](int r, int c) { return X + kW * c * kL + kW * r; };
-    const typename Mfma<T>::acc_t zero = {0, 0, 0, 0};
-    typename Mfma<T>::acc_t t = zero;  // L X product of the block of X that the wavefront forms next
+    tile_acc<T> t;  // L X product of the block of X that the wavefront forms next
+    clear<T>(t);
     // strip b beside work() on the wavefronts that have no rows in it; 0 or the failed pivot
-    auto pass = [&](auto strip, auto work) -> int {
+    auto pass = [&](auto strip, auto work) __attribute__((always_inline)) -> int {
         constexpr int b = decltype(strip)::value;
-        T diag[4];
+        real_t<T> diag[4][Field<T>::planes];
         if (wave < 4 - b) {
             const int f = factor_strip<T, b>(S, X, diag);
             if (threadIdx.x == 0) *s_flag = f;
         } else {
             work();
         }
+        if (b == 0) before();
         __syncthreads();
+        if (b == 0) after();
         if (wave == 0) store_diagonal<T>(diag, b, S);
         const int f = *s_flag;
         if (f != 0) __syncthreads();
@@ -347,7 +400,7 @@ __device__ __attribute__((always_inline)) inline int factor_invert64(T* S, T* X,
     int f = pass(Const<0>(), [] {});
     if (f != 0) return f;
     if (wave < 3) update_tile<T>(S, 0, 1 + wave, 1);
-    else t = tile_product<T>(s_at(1, 0), x_at(0, 0), zero);
+    else tile_product<T>(s_at(1, 0), x_at(0, 0), t);
     __syncthreads();
     f = pass(Const<1>(), [&] {
         update_tile<T>(S, 0, 2, 2);
@@ -359,11 +412,13 @@ __device__ __attribute__((always_inline)) inline int factor_invert64(T* S, T* X,
     else if (wave == 3) left_product<T>(x_at(1, 1), t, x_at(1, 0));
     __syncthreads();
     f = pass(Const<2>(), [&] {
+        clear<T>(t);
         if (wave == 2) {
-            t = tile_product<T>(s_at(2, 1), x_at(1, 0), tile_product<T>(s_at(2, 0), x_at(0, 0), zero));
+            tile_product<T>(s_at(2, 0), x_at(0, 0), t);
+            tile_product<T>(s_at(2, 1), x_at(1, 0), t);
         } else {
             update_tile<T>(S, 1, 3, 3);
-            t = tile_product<T>(s_at(2, 1), x_at(1, 1), zero);
+            tile_product<T>(s_at(2, 1), x_at(1, 1), t);
         }
     });
     if (f != 0) return f;
@@ -371,8 +426,8 @@ __device__ __attribute__((always_inline)) inline int factor_invert64(T* S, T* X,
     else if (wave > 1) left_product<T>(x_at(2, 2), t, x_at(2, wave - 2));
     __syncthreads();
     f = pass(Const<3>(), [&] {
-        t = zero;
-        for (int k = wave - 1; k < 3; ++k) t = tile_product<T>(s_at(3, k), x_at(k, wave - 1), t);
+        clear<T>(t);
+        for (int k = wave - 1; k < 3; ++k) tile_product<T>(s_at(3, k), x_at(k, wave - 1), t);
     });
     if (f != 0) return f;
     if (wave > 0) left_product<T>(x_at(3, 3), t, x_at(3, wave - 1));
@@ -380,47 +435,56 @@ __device__ __attribute__((always_inline)) inline int factor_invert64(T* S, T* X,
     return 0;
 }
 
+template <class T>
+__device__ __forceinline__ int factor_invert64(real_t<T>* S, real_t<T>* X, int* s_flag)
+{
+    return factor_invert64<T>(S, X, s_flag, [] {}, [] {});
+}
+
 // The same as an out-of-line function, for kernels whose register budget
 // cannot hold it inlined (it would spill there).
 template <class T>
-__device__ __attribute__((noinline)) int factor_invert64_call(T* S, T* X, int* s_flag)
+__device__ __attribute__((noinline)) int factor_invert64_call(real_t<T>* S, real_t<T>* X, int* s_flag)
 {
     return factor_invert64<T>(S, X, s_flag);
 }
 
 // Copies the referenced triangle of the w x w diagonal block at A (uplo
-// L: A[r + c * lda], r >= c; uplo U: A[c + r * lda]) into the lower triangle
-// of S, zeros above it and the identity beyond order w.
+// L: A[r + c * lda], r >= c; uplo U: conj(A[c + r * lda])) into the lower
+// triangle of S, zeros above it and the identity beyond order w.
 template <class T>
-__device__ void load_block(bool upper, int w, const T* A, long long lda, T* S)
+__device__ void load_block(bool upper, int w, const T* A, long long lda, real_t<T>* S)
 {
+    using R = real_t<T>;
 #pragma unroll 4
     for (int e = 0; e < kB * kB / 256; ++e) {
         const int idx = threadIdx.x + 256 * e;
         const int fast = idx & (kB - 1), slow = idx >> 6;
         const int r = upper ? slow : fast, c = upper ? fast : slow;
-        T v = T(0);
+        T v = element<T>(R(0), R(0));
         if (r < w && c < w) {
             if (r >= c) v = upper ? A[c + (long long)r * lda] : A[r + (long long)c * lda];
         } else if (r == c) {
-            v = T(1);
+            v = element<T>(R(1), R(0));
         }
-        S[c * kL + r] = v;
+        S[c * kL + r] = plane(v, 0);
+        if (Field<T>::planes == 2) S[kPlane + c * kL + r] = upper ? -plane(v, 1) : plane(v, 1);
     }
 }
 
 // Writes the lower triangle of S (order w) back to the referenced triangle at A.
 template <class T>
-__device__ void store_factor(bool upper, int w, const T* S, T* A, long long lda)
+__device__ void store_factor(bool upper, int w, const real_t<T>* S, T* A, long long lda)
 {
+    constexpr int last = (Field<T>::planes - 1) * kPlane;
 #pragma unroll 4
     for (int e = 0; e < kB * kB / 256; ++e) {
         const int idx = threadIdx.x + 256 * e;
         const int fast = idx & (kB - 1), slow = idx >> 6;
         const int r = upper ? slow : fast, c = upper ? fast : slow;
         if (r < w && c < w && r >= c) {
-            if (upper) A[c + (long long)r * lda] = S[c * kL + r];
-            else A[r + (long long)c * lda] = S[c * kL + r];
+            if (upper) A[c + (long long)r * lda] = element<T>(S[c * kL + r], -S[last + c * kL + r]);
+            else A[r + (long long)c * lda] = element<T>(S[c * kL + r], S[last + c * kL + r]);
         }
     }
 }
@@ -428,13 +492,14 @@ __device__ void store_factor(bool upper, int w, const T* S, T* A, long long lda)
 // Stores X as a full 64 x 64 column-major block (leading dimension 64) with
 // exact zeros above the diagonal.
 template <class T>
-__device__ void store_inverse(const T* X, T* inv)
+__device__ void store_inverse(const real_t<T>* X, T* inv)
 {
+    constexpr int last = (Field<T>::planes - 1) * kPlane;
 #pragma unroll 4
     for (int e = 0; e < kB * kB / 256; ++e) {
         const int idx = threadIdx.x + 256 * e;
         const int r = idx & (kB - 1), c = idx >> 6;
-        inv[idx] = r >= c ? X[c * kL + r] : T(0);
+        inv[idx] = r >= c ? element<T>(X[c * kL + r], X[last + c * kL + r]) : element<T>(0, 0);
     }
 }
 

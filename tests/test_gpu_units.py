@@ -1,0 +1,64 @@
+"""Factorizations at the edges of their blocks: orders around the 64-row blocks
+and the largest one-panel order (4096), the same matrix by narrow panels.
+
+Checked against the problem itself, in float64 on the GPU.  Tolerance: a
+backward-stable factorization has |A - L L^H|_F <= c n eps |A|_F with c a small
+constant times the condition of the inverted 64 x 64 diagonal blocks (below 5
+here: every spectrum lies in [0.5, 4.6]), so 10 n eps."""
+import numpy as np
+import pytest
+
+import libddla_amd as dd
+
+pytestmark = pytest.mark.gpu
+
+TORCH = {np.float64: "float64", np.float32: "float32", np.complex128: "complex128", np.complex64: "complex64"}
+
+
+def system(n, dtype, seed):
+    """Hermitian positive definite A in float64 / complex128 (rounded to dtype) on the GPU."""
+    import torch
+
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    wide = torch.complex128 if np.dtype(dtype).kind == "c" else torch.float64
+    g = torch.randn(n, n, dtype=wide, device="cuda", generator=gen)
+    a = torch.mm(g, g.mH.contiguous()) / n
+    a = (0.5 * (a + a.mH)).contiguous()
+    a.diagonal().add_(0.5)
+    return a.to(getattr(torch, TORCH[dtype])).to(wide), gen
+
+
+def factor(handle, a, dtype, uplo):
+    import torch
+
+    s = a.t().to(getattr(torch, TORCH[dtype])).clone(memory_format=torch.contiguous_format)  # column-major storage
+    torch.cuda.synchronize()
+    A = dd.DistributedMatrix.from_torch(handle, s, a.shape[0], a.shape[0])
+    assert dd.ppotrf(A, uplo)[1] == 0
+    return A, s
+
+
+def residual(a, s, uplo):
+    m = s.t().to(a.dtype)
+    low = m.tril() if uplo == "L" else m.triu().mH
+    import torch
+
+    return (torch.linalg.norm(a - torch.mm(low, low.mH.contiguous())) / torch.linalg.norm(a)).item()
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float64, n) for n in (65, 128, 191, 1000, 4032, 4096, 4160)] +
+                         [(np.float32, n) for n in (129, 1500, 4095, 4097)])
+@pytest.mark.parametrize("uplo", ["L", "U"])
+def test_factor_units(handle, dtype, n, uplo):
+    print(f"case units n={n} {np.dtype(dtype).name} {uplo}", flush=True)
+    a, _ = system(n, dtype, n)
+    tol = 10 * n * np.finfo(dtype).eps
+    A, s = factor(handle, a, dtype, uplo)
+    assert residual(a, s, uplo) <= tol
+    if n > 192:  # several panels with rows below them, updates between them
+        previous = dd.lib.ddla_c_set_panel_width(192)
+        try:
+            _, s2 = factor(handle, a, dtype, uplo)
+        finally:
+            dd.lib.ddla_c_set_panel_width(previous)
+        assert residual(a, s2, uplo) <= tol
