@@ -65,6 +65,10 @@ int outer_block(int n, bool split, bool one_panel = true)
 // brought there by potrf_blocked): element (i, j), i >= j, of L is
 // A[i + j*lda].  The helpers below translate operations on L into kernel
 // calls.
+// Real operations of one multiply-add term, over a real one's.
+template <class T>
+constexpr double kFlopsPerTerm = is_complex<T>::value ? 4 : 1;
+
 template <class T>
 struct LView {
     T* A;
@@ -80,10 +84,16 @@ void update_lower(DdlaStream* h, hipStream_t st, int cls, const LView<T>& v, int
                   bool mask, const int* abort, double flops, const kern::Batch& batch = kern::Batch())
 {
     if (M <= 0 || N <= 0) return;
-    LaunchTimer timer(h, cls, flops * batch.count, 0, st);
-    const bool lookahead = cls == kClassLookahead;
-    kern::gemm<T>(st, 'N', 'T', M, N, K, alpha, v.at(ai, ak), v.lda, v.at(bj, bk), v.lda, beta, v.at(ci, cj), v.lda,
-                  mask ? kTriLower : kTriNone, ci - cj, abort, lookahead, batch);
+    LaunchTimer timer(h, cls, flops * batch.count * kFlopsPerTerm<T>, 0, st);
+    if constexpr (is_complex<T>::value) {
+        kern::zgemm<typename real_type<T>::type>(st, true, true, 'N', 'C', M, N, K, alpha, v.at(ai, ak), v.lda,
+                                                 v.at(bj, bk), v.lda, beta, v.at(ci, cj), v.lda,
+                                                 mask ? kTriLower : kTriNone, ci - cj, abort);
+    } else {
+        const bool lookahead = cls == kClassLookahead;
+        kern::gemm<T>(st, 'N', 'T', M, N, K, alpha, v.at(ai, ak), v.lda, v.at(bj, bk), v.lda, beta, v.at(ci, cj),
+                      v.lda, mask ? kTriLower : kTriNone, ci - cj, abort, lookahead, batch);
+    }
 }
 
 // Factors the panel of columns [k, k + kb) of the order-n L view (its
@@ -94,7 +104,8 @@ void factor_panel(DdlaStream* h, hipStream_t st, const LView<T>& v, int n, int k
                   const kern::Batch& batch = kern::Batch())
 {
     const double below = (double)n - k - kb;
-    LaunchTimer timer(h, kClassPanel, ((double)kb * kb * kb / 3.0 + below * kb * kb) * batch.count, 0, st);
+    LaunchTimer timer(h, kClassPanel,
+                      ((double)kb * kb * kb / 3.0 + below * kb * kb) * batch.count * kFlopsPerTerm<T>, 0, st);
     kern::panel_factor<T>(st, n, v.A, v.lda, k, kb, info, work, batch);
 }
 
@@ -222,14 +233,16 @@ void potrf_blocked(DdlaStream* h, bool upper, int n, T* A, long long lda, int* i
         // triangle transposed) is factored, and the exchange is undone: the
         // factor lands in the upper triangle and the caller's strict lower
         // triangle is restored bit for bit (two HBM passes over the matrix).
-        const double bytes = 2.0 * n * (n - 1) * sizeof(T);
-        {
-            LaunchTimer timer(h, kClassOther, 0, bytes);
-            kern::swap_triangles<T>(h->stream, n, A, lda);
-        }
+        auto swap = [&]() {
+            LaunchTimer timer(h, kClassOther, 0, 2.0 * n * (n - 1) * sizeof(T));
+            if constexpr (is_complex<T>::value)
+                kern::zswap_triangles<typename real_type<T>::type>(h->stream, n, A, lda);
+            else
+                kern::swap_triangles<T>(h->stream, n, A, lda);
+        };
+        swap();
         potrf_blocked<T>(h, false, n, A, lda, info, work, split);
-        LaunchTimer timer(h, kClassOther, 0, bytes);
-        kern::swap_triangles<T>(h->stream, n, A, lda);
+        swap();
         return;
     }
     const LView<T> v{A, lda};
@@ -890,6 +903,10 @@ void potrf_blocked_dispatch(DdlaStream* h, bool upper, int n, T* A, long long ld
 }
 template void potrf_blocked_dispatch<float>(DdlaStream*, bool, int, float*, long long, int*, void*);
 template void potrf_blocked_dispatch<double>(DdlaStream*, bool, int, double*, long long, int*, void*);
+template void potrf_blocked_dispatch<std::complex<float>>(DdlaStream*, bool, int, std::complex<float>*, long long,
+                                                          int*, void*);
+template void potrf_blocked_dispatch<std::complex<double>>(DdlaStream*, bool, int, std::complex<double>*, long long,
+                                                           int*, void*);
 
 template <class T>
 void potrf_batched_dispatch(DdlaStream* h, int n, T* A, long long lda, int* info, void* work, const kern::Batch& batch)

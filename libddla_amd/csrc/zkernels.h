@@ -34,20 +34,21 @@ void zgemm_vbatched(hipStream_t s, bool a_complex, bool b_complex, char ta, char
                     const int* ldb, std::complex<R> beta, std::complex<R>* const* C, const int* ldc, int batch,
                     int max_m, int max_n);
 
-// Factors the order-w (w = min(64, n - k0)) Hermitian diagonal block at
-// A(k0, k0) in place (lower triangle: A = L L^H), writes its inverse L^-1 to
-// inv (64 x 64, column-major, zero above the diagonal) and, on a pivot whose
-// real part is not positive (or NaN), sets *info = k0 + j + 1 (1-based) and
-// leaves the block partly factored.  Does nothing if *info != 0 on entry.
-template <class R>
-void zpotf2(hipStream_t s, int n, std::complex<R>* A, long long lda, int k0, std::complex<R>* inv, int* info);
-
 // Inverse of every 64 x 64 diagonal block of the order-n lower factor L (L
 // view: L(i, j) = A[i + j lda], or conj(A[j + i lda]) when upper) into inv
 // (block b at inv + 4096 b).
 template <class R>
 void ztrtri_diag_blocks(hipStream_t s, bool upper, int n, const std::complex<R>* A, long long lda,
                         std::complex<R>* inv);
+
+// L Y = B, then L^H X = Y in place on B (n x nrhs) with the L view of A and its
+// inverted diagonal blocks dinv (ztrtri_diag_blocks): one persistent launch per
+// sweep.  sync: zsolve_sync_bytes(nrhs) bytes; *error is set to 1 if a wait
+// exceeds its limit.
+std::size_t zsolve_sync_bytes(int nrhs);
+template <class R>
+void zpotrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const std::complex<R>* A, long long lda,
+                   const std::complex<R>* dinv, std::complex<R>* B, long long ldb, void* sync, int* error);
 
 // out (n x m) = in^H (in m x n).
 template <class R>

@@ -6,15 +6,22 @@
 // (src/vbatched/gemm_template_kernel_vbatched.hpp:46-105,
 // src/diag_logdet_impl.h:50-113).
 //
-// Complex arithmetic runs on the vector ALUs: on MI355X the FP64 and FP32
-// vector FMA rates equal the matrix-core rates of those types (78.6 and
-// 157.3 TF/s), and a complex product is four real FMAs per lane with no
-// operand shuffling.  GEMM tiles are 64 x 64 per 256-thread workgroup, a 4 x 4
-// block of complex accumulators per thread, op(A) and op(B) staged through LDS
-// 16 columns deep with the next slab's loads in flight.
+// Complex products run on the matrix cores as products of real and imaginary
+// planes, four 16x16x4 steps for one of complex tiles (field.h); the planes are
+// parted when a slab is staged in LDS.  (On the vector ALUs, at the same peak
+// rates, every product also paid for its operands' LDS reads: 23 us for the
+// average trailing update of an FP64 order-2000 factorization, 64 columns deep.)
 #include "zkernels.h"
+#include "gemm_tile.h"
+#include "internal.h"
+#include "kernels.h"
+#include "panel_host.h"
+#include "panel_tile.h"
+#include "potf2_tile.h"
+#include "zsolve_tile.h"
 
 #include <cfloat>
+#include <climits>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -29,11 +36,6 @@ inline void zcheck_launch(const char* what)
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
-
-template <class R>
-struct Cx {
-    R re, im;
-};
 
 template <class R>
 __device__ __forceinline__ Cx<R> cmul(Cx<R> a, Cx<R> b)
@@ -55,12 +57,18 @@ __device__ __forceinline__ Cx<R> conj(Cx<R> a)
 }
 
 // ---------------------------------------------------------------------------
-// GEMM tile
+// GEMM tile: BM x BN of C per 256-thread workgroup, four wavefronts (2 x 2) of
+// (BM / 2) x (BN / 2), slabs of 16 columns of op(A) and rows of op(B) in LDS by
+// planes, the next slab's loads in flight while one is multiplied.
 // ---------------------------------------------------------------------------
-constexpr int kT = 64;   // tile rows / columns
+using gemm_detail::kPad;
+using gemm_detail::map_tile;
+using gemm_detail::Mfma;
+using gemm_detail::TileOrder;
+
+constexpr int kT = 64;   // rows and columns of a tile
 constexpr int kK = 16;   // slab depth
 constexpr int kTh = 256;
-constexpr int kPerT = kT * kK / kTh;  // operand elements per thread per slab (4)
 
 template <class R>
 struct ZProblem {
@@ -78,124 +86,174 @@ struct ZProblem {
     long long diag;
 };
 
-// Element of a real or complex operand (index idx of its array).
-template <class R, bool CPX>
-__device__ __forceinline__ Cx<R> operand(const void* P, long long idx, bool conjugate)
+// LDS elements of a tile's slabs (op(A)'s planes, then op(B)'s).
+template <int BM, int BN, bool ACPX, bool BCPX>
+constexpr int zslab_elems()
 {
-    if constexpr (CPX) {
-        const Cx<R> v = static_cast<const Cx<R>*>(P)[idx];
-        return conjugate ? Cx<R>{v.re, -v.im} : v;
-    } else {
-        return Cx<R>{static_cast<const R*>(P)[idx], R(0)};
-    }
+    return kK * ((ACPX ? 2 : 1) * (BM + kPad) + (BCPX ? 2 : 1) * (BN + kPad));
 }
 
-// Tile (ti, tj) of the problem.
-template <class R, bool ACPX, bool BCPX>
-__device__ void ztile(const ZProblem<R>& p, int ti, int tj, Cx<R> (*As)[kT + 1], Cx<R> (*Bs)[kT + 1])
+// One operand's slabs: D consecutive indices (rows of op(A) or columns of
+// op(B)) by kK of the inner dimension, for the tile at origin o of `extent`.
+// along: the stored contiguous dimension is the D one.  Loads of a slab that
+// reaches beyond the operand are clamped and dropped.
+template <class R, bool CPX, int D>
+struct ZOperand {
+    static constexpr int PER = D * kK / kTh, LD = D + kPad;
+    using E = std::conditional_t<CPX, Cx<R>, R>;
+    const E* P;
+    long long ld;
+    int o, extent, k;
+    bool along, conjugate;
+    E v[PER];
+    __device__ int index(int e) const { const int i = threadIdx.x + kTh * e; return along ? i % D : i / kK; }
+    __device__ int inner(int e) const { const int i = threadIdx.x + kTh * e; return along ? i / D : i % kK; }
+    __device__ void load(int k0)
+    {
+        if (o + D <= extent && k0 + kK <= k) {
+            const E* base = P + (along ? o + k0 * ld : k0 + o * ld);
+#pragma unroll
+            for (int e = 0; e < PER; ++e) v[e] = base[along ? index(e) + inner(e) * ld : inner(e) + index(e) * ld];
+        } else {
+#pragma unroll
+            for (int e = 0; e < PER; ++e) {
+                const int i = o + index(e), kk = k0 + inner(e);
+                const long long ci = min(i, extent - 1), ck = min(kk, k - 1);
+                const E x = P[along ? ci + ck * ld : ck + ci * ld];
+                v[e] = i < extent && kk < k ? x : E{};
+            }
+        }
+    }
+    __device__ void store(R* S) const
+    {
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            R* p = S + inner(e) * LD + index(e);
+            if constexpr (CPX) {
+                p[0] = v[e].re;
+                p[kK * LD] = conjugate ? -v[e].im : v[e].im;
+            } else {
+                p[0] = v[e];
+            }
+        }
+    }
+};
+
+template <class R, int BM, int BN, bool ACPX, bool BCPX>
+__device__ void ztile(const ZProblem<R>& p, int ti, int tj, R* smem)
 {
-    const int m0 = ti * kT, n0 = tj * kT;
+    using Op = Mfma<R>;
+    constexpr int TM = BM / 32, TN = BN / 32;
+    const int m0 = ti * BM, n0 = tj * BN;
     if (m0 >= p.m || n0 >= p.n) return;
-    if (p.tri == 1 && (long long)(m0 + kT - 1) + p.diag < n0) return;  // wholly above the written lower part
-    if (p.tri == 2 && (long long)m0 + p.diag > n0 + kT - 1) return;    // wholly below the written upper part
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    Cx<R> acc[4][4];
+    if (p.tri == 1 && (long long)(m0 + BM - 1) + p.diag < n0) return;  // wholly above the written lower part
+    if (p.tri == 2 && (long long)m0 + p.diag > n0 + BN - 1) return;    // wholly below the written upper part
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+    // D^T = op(B)^T op(A)^T: lane l % 16 of an accumulator runs along i, C's contiguous dimension
+    // The terms add up 64 at a time (acc, then into sum): C's scale rounds once in
+    // 64 terms, as in a factorization by block columns of 64.
+    typename Op::acc_t acc[TM][TN][2], sum[TM][TN][2];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int x = 0; x < TM; ++x)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = Cx<R>{R(0), R(0)};
-    const bool product = p.k > 0 && (p.alpha.re != R(0) || p.alpha.im != R(0));
-    if (product) {
-        const bool a_n = p.opa == 0, b_n = p.opb == 0;
-        const bool a_conj = p.opa == 2, b_conj = p.opb == 2;
-        Cx<R> va[kPerT], vb[kPerT];
-        // op(A)(i, kk) and op(B)(kk, j) of slab k0, clamped and masked
-        auto load = [&](int k0) {
+        for (int y = 0; y < TN; ++y)
 #pragma unroll
-            for (int e = 0; e < kPerT; ++e) {
-                const int idx = tid + kTh * e;
-                const int i = a_n ? (idx & (kT - 1)) : (idx >> 4);
-                const int kk = a_n ? (idx >> 6) : (idx & (kK - 1));
-                const int gi = m0 + i, gk = k0 + kk;
-                const bool in = gi < p.m && gk < p.k;
-                const long long ci = min(gi, p.m - 1), ck = min(gk, p.k - 1);
-                const Cx<R> v = operand<R, ACPX>(p.A, a_n ? ci + ck * p.lda : ck + ci * p.lda, a_conj);
-                va[e] = in ? v : Cx<R>{R(0), R(0)};
-            }
-#pragma unroll
-            for (int e = 0; e < kPerT; ++e) {
-                const int idx = tid + kTh * e;
-                const int kk = b_n ? (idx & (kK - 1)) : (idx >> 6);
-                const int j = b_n ? (idx >> 4) : (idx & (kT - 1));
-                const int gj = n0 + j, gk = k0 + kk;
-                const bool in = gj < p.n && gk < p.k;
-                const long long cj = min(gj, p.n - 1), ck = min(gk, p.k - 1);
-                const Cx<R> v = operand<R, BCPX>(p.B, b_n ? ck + cj * p.ldb : cj + ck * p.ldb, b_conj);
-                vb[e] = in ? v : Cx<R>{R(0), R(0)};
-            }
-        };
-        auto store = [&]() {
-#pragma unroll
-            for (int e = 0; e < kPerT; ++e) {
-                const int idx = tid + kTh * e;
-                const int i = a_n ? (idx & (kT - 1)) : (idx >> 4);
-                const int kk = a_n ? (idx >> 6) : (idx & (kK - 1));
-                As[kk][i] = va[e];
-            }
-#pragma unroll
-            for (int e = 0; e < kPerT; ++e) {
-                const int idx = tid + kTh * e;
-                const int kk = b_n ? (idx & (kK - 1)) : (idx >> 6);
-                const int j = b_n ? (idx >> 4) : (idx & (kT - 1));
-                Bs[kk][j] = vb[e];
-            }
-        };
-        load(0);
+            for (int c = 0; c < 2; ++c) acc[x][y][c] = sum[x][y][c] = typename Op::acc_t{0, 0, 0, 0};
+    if (p.k > 0 && (p.alpha.re != R(0) || p.alpha.im != R(0))) {
+        using OpA = ZOperand<R, ACPX, BM>;
+        using OpB = ZOperand<R, BCPX, BN>;
+        OpA a{static_cast<const typename OpA::E*>(p.A), p.lda, m0, p.m, p.k, p.opa == 0, p.opa == 2, {}};
+        OpB b{static_cast<const typename OpB::E*>(p.B), p.ldb, n0, p.n, p.k, p.opb != 0, p.opb == 2, {}};
+        R* const As = smem;
+        R* const Bs = smem + (ACPX ? 2 : 1) * kK * OpA::LD;
+        a.load(0);
+        b.load(0);
         for (int k0 = 0; k0 < p.k; k0 += kK) {
-            store();
+            a.store(As);
+            b.store(Bs);
             __syncthreads();
-            if (k0 + kK < p.k) load(k0 + kK);
-#pragma unroll 4
-            for (int kk = 0; kk < kK; ++kk) {
-                Cx<R> a[4], b[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) a[r] = As[kk][tx * 4 + r];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) b[c] = Bs[kk][ty * 4 + c];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) cfma(acc[r][c], a[r], b[c]);
+            if (k0 + kK < p.k) {
+                a.load(k0 + kK);
+                b.load(k0 + kK);
             }
+#pragma unroll
+            for (int kk = 0; kk < kK; kk += 4) {
+                const R* ap = As + (kk + lk) * OpA::LD + wm + li;
+                const R* bp = Bs + (kk + lk) * OpB::LD + wn + li;
+                R ar[TM], ai[TM], br[TN], bi[TN];
+#pragma unroll
+                for (int x = 0; x < TM; ++x) {
+                    ar[x] = ap[16 * x];
+                    if (ACPX) ai[x] = ap[kK * OpA::LD + 16 * x];
+                }
+#pragma unroll
+                for (int y = 0; y < TN; ++y) {
+                    br[y] = bp[16 * y];
+                    if (BCPX) bi[y] = bp[kK * OpB::LD + 16 * y];
+                }
+#pragma unroll
+                for (int x = 0; x < TM; ++x)
+#pragma unroll
+                    for (int y = 0; y < TN; ++y) {
+                        acc[x][y][0] = Op::mma(br[y], ar[x], acc[x][y][0]);
+                        if (ACPX) acc[x][y][1] = Op::mma(br[y], ai[x], acc[x][y][1]);
+                        if (ACPX && BCPX) acc[x][y][0] = Op::mma(bi[y], -ai[x], acc[x][y][0]);
+                        if (BCPX) acc[x][y][1] = Op::mma(bi[y], ar[x], acc[x][y][1]);
+                    }
+            }
+            if ((k0 + kK) % 64 == 0 || k0 + kK >= p.k)
+#pragma unroll
+                for (int x = 0; x < TM; ++x)
+#pragma unroll
+                    for (int y = 0; y < TN; ++y)
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            sum[x][y][c] += acc[x][y][c];
+                            acc[x][y][c] = typename Op::acc_t{0, 0, 0, 0};
+                        }
             __syncthreads();
         }
     }
+    // Accumulator (x, y, r) of lane l: i = 16 x + l % 16, j = 16 y + row(l, r)
+    // within the wavefront's block.  A row of blocks of C is read before it is
+    // written, so that its reads are in flight together.
     const bool beta_zero = p.beta.re == R(0) && p.beta.im == R(0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int j = n0 + ty * 4 + c;
-        if (j >= p.n) continue;
+    for (int x = 0; x < TM; ++x) {
+        const int i = m0 + wm + 16 * x + li;
+        Cx<R> cv[TN][4];
+        bool live[TN][4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = m0 + tx * 4 + r;
-            if (i >= p.m) continue;
-            if (p.tri == 1 && (long long)i + p.diag < j) continue;
-            if (p.tri == 2 && (long long)i + p.diag > j) continue;
-            Cx<R>* cp = p.C + i + (long long)j * p.ldc;
-            Cx<R> v = cmul(p.alpha, acc[r][c]);
-            if (!beta_zero) cfma(v, p.beta, *cp);
-            *cp = v;
-        }
+        for (int y = 0; y < TN; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int j = n0 + wn + 16 * y + Op::row(lane, r);
+                live[y][r] = i < p.m && j < p.n && (p.tri != 1 || (long long)i + p.diag >= j) &&
+                             (p.tri != 2 || (long long)i + p.diag <= j);
+                cv[y][r] = Cx<R>{R(0), R(0)};
+                if (!beta_zero && live[y][r]) cv[y][r] = p.C[i + (long long)j * p.ldc];
+            }
+#pragma unroll
+        for (int y = 0; y < TN; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int j = n0 + wn + 16 * y + Op::row(lane, r);
+                Cx<R> v = cmul(p.alpha, Cx<R>{sum[x][y][0][r], sum[x][y][1][r]});
+                if (!beta_zero) cfma(v, p.beta, cv[y][r]);
+                if (live[y][r]) p.C[i + (long long)j * p.ldc] = v;
+            }
     }
 }
 
-template <class R, bool ACPX, bool BCPX>
-__global__ __launch_bounds__(kTh) void zgemm_kernel(ZProblem<R> p, const int* abort)
+template <class R, int BM, int BN, bool ACPX, bool BCPX>
+__global__ __launch_bounds__(kTh, 2) void zgemm_kernel(ZProblem<R> p, TileOrder o, const int* abort)
 {
-    __shared__ Cx<R> As[kK][kT + 1];
-    __shared__ Cx<R> Bs[kK][kT + 1];
+    __shared__ R smem[zslab_elems<BM, BN, ACPX, BCPX>()];
     if (abort != nullptr && *abort != 0) return;
-    ztile<R, ACPX, BCPX>(p, blockIdx.x, blockIdx.y, As, Bs);
+    int ti, tj;
+    if (!map_tile(o, blockIdx.x, ti, tj)) return;
+    ztile<R, BM, BN, ACPX, BCPX>(p, ti, tj, smem);
 }
 
 template <class R>
@@ -209,10 +267,9 @@ struct ZBatch {
 };
 
 template <class R, bool ACPX, bool BCPX>
-__global__ __launch_bounds__(kTh) void zgemm_vbatched_kernel(ZBatch<R> v)
+__global__ __launch_bounds__(kTh, 2) void zgemm_vbatched_kernel(ZBatch<R> v)
 {
-    __shared__ Cx<R> As[kK][kT + 1];
-    __shared__ Cx<R> Bs[kK][kT + 1];
+    __shared__ R smem[zslab_elems<kT, kT, ACPX, BCPX>()];
     const int b = v.z0 + blockIdx.z;
     if (b >= v.batch) return;
     ZProblem<R> p;
@@ -232,124 +289,22 @@ __global__ __launch_bounds__(kTh) void zgemm_vbatched_kernel(ZBatch<R> v)
     p.ldc = v.ldc[b];
     p.tri = 0;
     p.diag = 0;
-    ztile<R, ACPX, BCPX>(p, blockIdx.x, blockIdx.y, As, Bs);
+    ztile<R, kT, kT, ACPX, BCPX>(p, blockIdx.x, blockIdx.y, smem);
 }
 
-// ---------------------------------------------------------------------------
-// 64 x 64 Hermitian diagonal block: factor (lower, right-looking, in LDS) and
-// inverse of the factor.
-// ---------------------------------------------------------------------------
-constexpr int kD = 64;
-constexpr int kDL = kD + 1;
-
-// X := S^-1 for the order-w lower-triangular S (real positive diagonal) in
-// LDS; thread c < 64 forms column c by forward substitution.  Rows and
-// columns from w on: X = identity there.
-template <class R>
-__device__ void invert_lower(int w, Cx<R> (*S)[kDL], Cx<R> (*X)[kDL])
-{
-    const int c = threadIdx.x;
-    if (c < kD) {
-        for (int i = 0; i < kD; ++i) {
-            if (i < c || c >= w || i >= w) {
-                X[i][c] = Cx<R>{(i == c) ? R(1) : R(0), R(0)};
-                continue;
-            }
-            Cx<R> acc{i == c ? R(1) : R(0), R(0)};
-            for (int k = c; k < i; ++k) {
-                const Cx<R> l = S[i][k], x = X[k][c];
-                acc.re -= l.re * x.re - l.im * x.im;
-                acc.im -= l.re * x.im + l.im * x.re;
-            }
-            const R d = S[i][i].re;
-            X[i][c] = Cx<R>{acc.re / d, acc.im / d};
-        }
-    }
-}
-
-template <class R>
-__device__ void store_inverse(Cx<R> (*X)[kDL], Cx<R>* inv)
-{
-    for (int idx = threadIdx.x; idx < kD * kD; idx += blockDim.x) {
-        const int r = idx & (kD - 1), c = idx >> 6;
-        inv[idx] = r >= c ? X[r][c] : Cx<R>{R(0), R(0)};
-    }
-}
-
-template <class R>
-__global__ __launch_bounds__(256) void zpotf2_kernel(int n, Cx<R>* A, long long lda, int k0, Cx<R>* inv, int* info)
-{
-    __shared__ Cx<R> S[kD][kDL];
-    __shared__ Cx<R> X[kD][kDL];
-    __shared__ int s_fail;
-    if (*info != 0) return;
-    const int w = min(kD, n - k0), tid = threadIdx.x;
-    Cx<R>* D = A + k0 + (long long)k0 * lda;
-    for (int idx = tid; idx < kD * kD; idx += 256) {
-        const int r = idx & (kD - 1), c = idx >> 6;
-        S[r][c] = (r < w && c < w && r >= c) ? D[r + (long long)c * lda] : Cx<R>{R(0), R(0)};
-    }
-    if (tid == 0) s_fail = 0;
-    __syncthreads();
-    for (int j = 0; j < w; ++j) {
-        const R d = S[j][j].re;
-        if (!(d > R(0))) {  // not positive, or NaN (LAPACK zpotrf's test on the real diagonal)
-            if (tid == 0) s_fail = j + 1;
-            break;  // uniform: every thread reads the same S[j][j]
-        }
-        const R l = sqrt(d);
-        __syncthreads();
-        if (tid == 0) S[j][j] = Cx<R>{l, R(0)};
-        for (int i = j + 1 + tid; i < w; i += 256) S[i][j] = Cx<R>{S[i][j].re / l, S[i][j].im / l};
-        __syncthreads();
-        // S(i, c) -= S(i, j) conj(S(c, j)), j < c <= i < w
-        const int t = w - j - 1;
-        for (int idx = tid; idx < t * t; idx += 256) {
-            const int ii = idx % t, cc = idx / t;
-            if (ii < cc) continue;
-            const int i = j + 1 + ii, c = j + 1 + cc;
-            const Cx<R> a = S[i][j], b = S[c][j];
-            S[i][c].re -= a.re * b.re + a.im * b.im;
-            S[i][c].im -= a.im * b.re - a.re * b.im;
-        }
-        __syncthreads();
-    }
-    __syncthreads();
-    // the factored part (and, on failure, the partly updated rest) goes back
-    for (int idx = tid; idx < kD * kD; idx += 256) {
-        const int r = idx & (kD - 1), c = idx >> 6;
-        if (r < w && c < w && r >= c) D[r + (long long)c * lda] = S[r][c];
-    }
-    if (s_fail != 0) {
-        if (tid == 0) *info = k0 + s_fail;
-        return;
-    }
-    invert_lower<R>(w, S, X);
-    __syncthreads();
-    store_inverse<R>(X, inv);
-}
-
+// inv(block b) = L(b, b)^-1 for every 64 x 64 diagonal block of a factor.
 template <class R>
 __global__ __launch_bounds__(256) void ztrtri_kernel(bool upper, int n, const Cx<R>* A, long long lda, Cx<R>* inv)
 {
-    __shared__ Cx<R> S[kD][kDL];
-    __shared__ Cx<R> X[kD][kDL];
-    const long long k0 = (long long)blockIdx.x * kD;
-    const int w = (int)min((long long)kD, n - k0);
-    for (int idx = threadIdx.x; idx < kD * kD; idx += 256) {
-        const int r = idx & (kD - 1), c = idx >> 6;
-        Cx<R> v{R(0), R(0)};
-        if (r < w && c < w && r >= c) {
-            // L view: L(i, j) = A[i + j lda], or conj(A[j + i lda]) for an upper factor
-            const long long i = k0 + r, j = k0 + c;
-            v = upper ? conj(A[j + i * lda]) : A[i + j * lda];
-        }
-        S[r][c] = v;
-    }
+    using namespace potf2_detail;
+    __shared__ R S[2 * kPlane], X[2 * kPlane], rdiag[kB];
+    const long long j0 = (long long)blockIdx.x * kB;
+    load_block<Cx<R>>(upper, (int)min((long long)kB, n - j0), A + j0 + j0 * lda, lda, S);
     __syncthreads();
-    invert_lower<R>(w, S, X);
+    if (threadIdx.x < kB) rdiag[threadIdx.x] = R(1) / S[threadIdx.x * kL + threadIdx.x];
     __syncthreads();
-    store_inverse<R>(X, inv + (long long)blockIdx.x * kD * kD);
+    invert_lower<Cx<R>>(S, rdiag, X);
+    store_inverse<Cx<R>>(X, inv + (long long)blockIdx.x * kB * kB);
 }
 
 // ---------------------------------------------------------------------------
@@ -471,14 +426,22 @@ __global__ void zlogdet_final_kernel(const double* pmag, const double* pphase, c
     *reinterpret_cast<int*>(out + 2) = f;
 }
 
-template <class R>
+template <class R, int BM, int BN>
 void launch_zgemm(hipStream_t s, bool ac, bool bc, const ZProblem<R>& p, const int* abort)
 {
-    const dim3 grid((unsigned)((p.m + kT - 1) / kT), (unsigned)((p.n + kT - 1) / kT));
-    if (grid.y > 65535) throw std::invalid_argument("zgemm: too many column tiles");
-    if (ac && bc) zgemm_kernel<R, true, true><<<grid, kTh, 0, s>>>(p, abort);
-    else if (ac) zgemm_kernel<R, true, false><<<grid, kTh, 0, s>>>(p, abort);
-    else if (bc) zgemm_kernel<R, false, true><<<grid, kTh, 0, s>>>(p, abort);
+    TileOrder o;
+    o.ntm = (p.m + BM - 1) / BM;
+    o.ntn = (p.n + BN - 1) / BN;
+    o.lower_enum = (p.tri == 1 && p.diag == 0 && p.m == p.n && BM == BN) ? 1 : 0;
+    const long long total = o.lower_enum ? (long long)o.ntm * (o.ntm + 1) / 2 : (long long)o.ntm * o.ntn;
+    if (total > (long long)INT_MAX / 2) throw std::invalid_argument("zgemm: problem too large for one launch");
+    o.total = (int)total;
+    o.group = 8;
+    o.per_xcd = (o.total + 7) / 8;
+    const unsigned grid = (unsigned)(o.per_xcd * 8);
+    if (ac && bc) zgemm_kernel<R, BM, BN, true, true><<<grid, kTh, 0, s>>>(p, o, abort);
+    else if (ac) zgemm_kernel<R, BM, BN, true, false><<<grid, kTh, 0, s>>>(p, o, abort);
+    else if (bc) zgemm_kernel<R, BM, BN, false, true><<<grid, kTh, 0, s>>>(p, o, abort);
     else throw std::invalid_argument("zgemm: at least one complex operand");
     zcheck_launch("zgemm");
 }
@@ -517,7 +480,7 @@ void zgemm(hipStream_t s, bool a_complex, bool b_complex, char ta, char tb, int 
     p.ldc = ldc;
     p.tri = tri;
     p.diag = diag;
-    launch_zgemm<R>(s, a_complex, b_complex, p, abort);
+    launch_zgemm<R, kT, kT>(s, a_complex, b_complex, p, abort);
 }
 
 template <class R>
@@ -556,21 +519,37 @@ void zgemm_vbatched(hipStream_t s, bool a_complex, bool b_complex, char ta, char
 }
 
 template <class R>
-void zpotf2(hipStream_t s, int n, std::complex<R>* A, long long lda, int k0, std::complex<R>* inv, int* info)
-{
-    zpotf2_kernel<R><<<1, 256, 0, s>>>(n, reinterpret_cast<Cx<R>*>(A), lda, k0, reinterpret_cast<Cx<R>*>(inv),
-                                       info);
-    zcheck_launch("zpotf2");
-}
-
-template <class R>
 void ztrtri_diag_blocks(hipStream_t s, bool upper, int n, const std::complex<R>* A, long long lda,
                         std::complex<R>* inv)
 {
     if (n <= 0) return;
-    ztrtri_kernel<R><<<(n + kD - 1) / kD, 256, 0, s>>>(upper, n, reinterpret_cast<const Cx<R>*>(A), lda,
-                                                       reinterpret_cast<Cx<R>*>(inv));
+    ztrtri_kernel<R><<<(n + 63) / 64, 256, 0, s>>>(upper, n, reinterpret_cast<const Cx<R>*>(A), lda,
+                                                   reinterpret_cast<Cx<R>*>(inv));
     zcheck_launch("ztrtri_diag_blocks");
+}
+
+std::size_t zsolve_sync_bytes(int nrhs)
+{
+    return ((std::size_t)zsolve_detail::slabs(nrhs) * 4 * sizeof(int) + 255) / 256 * 256;
+}
+
+template <class R>
+void zpotrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const std::complex<R>* A, long long lda,
+                   const std::complex<R>* dinv, std::complex<R>* B, long long ldb, void* sync, int* error)
+{
+    using namespace zsolve_detail;
+    if (n <= 0 || nrhs <= 0) return;
+    const int ns = slabs(nrhs);
+    if (ns > 65535) throw std::invalid_argument("zpotrs_sweeps: too many right-hand sides");
+    SweepArgs<R> a{n, nrhs, (n + kSB - 1) / kSB, reinterpret_cast<const Cx<R>*>(A), lda, upper ? 1 : 0,
+                   reinterpret_cast<const Cx<R>*>(dinv), reinterpret_cast<Cx<R>*>(B), ldb, static_cast<int*>(sync),
+                   error, wait_limit()};
+    zero_counters_kernel<<<1, 256, 0, s>>>(a.sync, 4 * ns);
+    const dim3 grid((unsigned)a.nblk, (unsigned)ns);
+    sweep_kernel<R, false><<<grid, kSThreads, 0, s>>>(a);
+    a.sync += 2 * ns;
+    sweep_kernel<R, true><<<grid, kSThreads, 0, s>>>(a);
+    zcheck_launch("zpotrs_sweeps");
 }
 
 template <class R>
@@ -618,7 +597,13 @@ void zdiag_logdet(hipStream_t s, int n, const std::complex<R>* A, long long lda,
                                     std::complex<R>, const void* const*, const int*, const void* const*,         \
                                     const int*, std::complex<R>, std::complex<R>* const*, const int*, int, int,  \
                                     int);                                                                        \
-    template void zpotf2<R>(hipStream_t, int, std::complex<R>*, long long, int, std::complex<R>*, int*);         \
+    template void zpotrs_sweeps<R>(hipStream_t, bool, int, int, const std::complex<R>*, long long,               \
+                                   const std::complex<R>*, std::complex<R>*, long long, void*, int*);            \
+    template size_t panel_work_bytes<std::complex<R>>(int);                                                      \
+    template void panel_reset<std::complex<R>>(hipStream_t, int, void*, const Batch&);                           \
+    template int* panel_error_word<std::complex<R>>(int, void*);                                                 \
+    template void panel_factor<std::complex<R>>(hipStream_t, int, std::complex<R>*, long long, int, int, int*,   \
+                                                void*, const Batch&);                                            \
     template void ztrtri_diag_blocks<R>(hipStream_t, bool, int, const std::complex<R>*, long long,              \
                                         std::complex<R>*);                                                       \
     template void zconj_transpose<R>(hipStream_t, int, int, const std::complex<R>*, long long, std::complex<R>*, \

@@ -1,5 +1,6 @@
 """Factorizations at the edges of their blocks: orders around the 64-row blocks
-and the largest one-panel order (4096), the same matrix by narrow panels.
+and the largest one-panel order (4096), the same matrix by narrow panels, and complex
+elements.
 
 Checked against the problem itself, in float64 on the GPU.  Tolerance: a
 backward-stable factorization has |A - L L^H|_F <= c n eps |A|_F with c a small
@@ -47,7 +48,9 @@ def residual(a, s, uplo):
 
 
 @pytest.mark.parametrize("dtype,n", [(np.float64, n) for n in (65, 128, 191, 1000, 4032, 4096, 4160)] +
-                         [(np.float32, n) for n in (129, 1500, 4095, 4097)])
+                         [(np.float32, n) for n in (129, 1500, 4095, 4097)] +
+                         [(np.complex128, n) for n in (1, 63, 65, 200, 1025)] +
+                         [(np.complex64, n) for n in (64, 130, 1500, 4161)])
 @pytest.mark.parametrize("uplo", ["L", "U"])
 def test_factor_units(handle, dtype, n, uplo):
     print(f"case units n={n} {np.dtype(dtype).name} {uplo}", flush=True)
