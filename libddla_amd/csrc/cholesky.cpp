@@ -289,27 +289,6 @@ void potrf_blocked(DdlaStream* h, bool upper, int n, T* A, long long lda, int* i
     }
 }
 
-// Left solve A X = B with A = L L^T given by its L view; B is n x nrhs: the
-// forward and the backward sweep, one launch each.  stage_work (optional):
-// the staged solve's work (kern::stage_work_bytes), used when
-// kern::stage_solve(n, nrhs).
-template <class T>
-void solve_left(DdlaStream* h, bool upper, int n, int nrhs, const T* F, long long ldf, T* B, long long ldb,
-                const T* dinv, void* sync, int* error, void* stage_work)
-{
-    if (stage_work != nullptr && kern::stage_solve(n, nrhs)) {
-        {
-            LaunchTimer timer(h, kClassTrtri, 2.0 * n * 512.0 * 512.0 + (double)n * 512.0 * 512.0 / 3.0);
-            kern::stage_prepare<T>(h->stream, upper, n, F, ldf, dinv, stage_work);
-        }
-        LaunchTimer timer(h, kClassSolve, 2.0 * n * n * nrhs, (double)n * n * sizeof(T));
-        kern::stage_sweeps<T>(h->stream, upper, n, nrhs, F, ldf, B, ldb, stage_work, error);
-        return;
-    }
-    LaunchTimer timer(h, kClassSolve, 2.0 * n * n * nrhs, (double)n * n * sizeof(T));
-    kern::potrs_sweeps<T>(h->stream, upper, n, nrhs, F, ldf, dinv, B, ldb, sync, error);
-}
-
 std::size_t diag_inverse_elems(int n) { return (std::size_t)((n + kIB - 1) / kIB) * kIB * kIB; }
 
 void bad_workspace(const char* who)
@@ -400,17 +379,20 @@ void ppotrs_check(const DdlaHandle_t& h, char side, char uplo, char trans, int n
     if (rows && cols && !B) throw std::invalid_argument("ppotrs: null local right-hand side");
 }
 
-// Backend bytes of a ppotrs run; staged: with the staged solve's work when
-// the order and right-hand sides take that route.
+// Backend bytes of a ppotrs run.  wide: where the order and right-hand sides
+// allow it, over 128-row blocks (kern::wide_solve), whose work grows by n * 128
+// elements; otherwise the 64-row sweeps.
 template <class T>
-std::size_t ppotrs_bytes(char side, int n, int nrhs, bool staged)
+std::size_t ppotrs_bytes(char side, int n, int nrhs, bool wide)
 {
     if (n == 0 || nrhs == 0) return 0;
-    // [ inverses of the 64 x 64 diagonal blocks | sweep counters | error word | staged-solve work |
+    // [ error word | wide solve's work, or: inverses of the 64 x 64 diagonal blocks | sweep counters |
     //   transposed B (side 'R') ]
-    std::size_t b = detail::padded_bytes<T>(diag_inverse_elems(n)) + kern::solve_work_bytes(nrhs) +
-                    detail::padded_bytes<int>(1);
-    if (staged) b += detail::padded_bytes<char>(kern::stage_work_bytes(n, nrhs, sizeof(T)));
+    std::size_t b = detail::padded_bytes<int>(1);
+    if (wide && kern::wide_solve(n, nrhs, sizeof(T)))
+        b += detail::padded_bytes<char>(kern::wide_work_bytes(n, nrhs, sizeof(T)));
+    else
+        b += detail::padded_bytes<T>(diag_inverse_elems(n)) + kern::solve_work_bytes(nrhs);
     if (side == 'R') b += detail::padded_bytes<T>((std::size_t)n * nrhs);
     return b;
 }
@@ -428,33 +410,44 @@ void ppotrs_workspace_size(const DdlaHandle_t&, char side, int n, int nrhs, cons
 
 template <class T>
 void ppotrs_exec(const DdlaHandle_t& h, char side, char uplo, int n, int nrhs, const T* A, const int* da, T* B,
-                 const int* db, void* backend_work, std::size_t backend_bytes, bool staged)
+                 const int* db, void* backend_work, std::size_t backend_bytes, bool wide)
 {
     if (n == 0 || nrhs == 0) return;
-    if (backend_bytes < ppotrs_bytes<T>(side, n, nrhs, staged) || backend_work == nullptr) bad_workspace("ppotrs");
+    if (backend_bytes < ppotrs_bytes<T>(side, n, nrhs, wide) || backend_work == nullptr) bad_workspace("ppotrs");
     const bool upper = uplo == 'U';
     const long long lda = da[DDLA_LLD_], ldb = db[DDLA_LLD_];
     char* w = static_cast<char*>(backend_work);
-    T* dinv = detail::take<T>(w, diag_inverse_elems(n));
-    void* sync = w;
-    w += kern::solve_work_bytes(nrhs);
     int* error = detail::take<int>(w, 1);
-    void* stage_work = nullptr;
-    if (staged && kern::stage_solve(n, nrhs))
-        stage_work = detail::take<char>(w, kern::stage_work_bytes(n, nrhs, sizeof(T)));
     fill_int(h->stream, error, 0);
-    {
+    wide = wide && kern::wide_solve(n, nrhs, sizeof(T));
+    void* wide_work = nullptr;
+    T* dinv = nullptr;
+    void* sync = nullptr;
+    if (wide) {
+        wide_work = detail::take<char>(w, kern::wide_work_bytes(n, nrhs, sizeof(T)));
+        LaunchTimer timer(h, kClassTrtri, (double)n * 128 * 128 / 3.0);
+        kern::wide_prepare<T>(h->stream, upper, n, A, lda, wide_work);
+    } else {
+        dinv = detail::take<T>(w, diag_inverse_elems(n));
+        sync = w;
+        w += kern::solve_work_bytes(nrhs);
         LaunchTimer timer(h, kClassTrtri, (double)n * kIB * kIB / 3.0);
         kern::trtri_diag_blocks<T>(h->stream, upper, n, A, lda, dinv);
     }
+    // the forward and the backward sweep, A = L L^T given by its L view
+    auto sweeps = [&](T* X, long long ldx) {
+        LaunchTimer timer(h, kClassSolve, 2.0 * n * n * nrhs, (double)n * n * sizeof(T));
+        if (wide) kern::wide_sweeps<T>(h->stream, upper, n, nrhs, A, lda, X, ldx, wide_work, error);
+        else kern::potrs_sweeps<T>(h->stream, upper, n, nrhs, A, lda, dinv, X, ldx, sync, error);
+    };
     // A = L L^T is symmetric: trans 'N' and 'C' solve the same system.
     // side 'R' (X A = B, B nrhs x n) is A X^T = B^T.
     if (side == 'L') {
-        solve_left<T>(h, upper, n, nrhs, A, lda, B, ldb, dinv, sync, error, stage_work);
+        sweeps(B, ldb);
     } else {
         T* bt = detail::take<T>(w, (std::size_t)n * nrhs);
         kern::transpose<T>(h->stream, nrhs, n, B, ldb, bt, n);
-        solve_left<T>(h, upper, n, nrhs, A, lda, bt, n, dinv, sync, error, stage_work);
+        sweeps(bt, n);
         kern::transpose<T>(h->stream, n, nrhs, bt, n, B, ldb);
     }
     int host_error = 0;
@@ -511,16 +504,16 @@ void pposv_run(const DdlaHandle_t& h, char side, char uplo, char trans, int n, i
 } // namespace cholesky_impl
 
 template <class T>
-std::size_t pposv_unstaged_bytes(char side, int n, int nrhs)
+std::size_t pposv_bytes(char side, int n, int nrhs, bool wide)
 {
     std::size_t fb = 0, fh = 0;
     cholesky_impl::ppotrf_workspace_size<T>(nullptr, 'L', n, static_cast<T*>(nullptr), nullptr, &fb, &fh);
-    return std::max(fb, cholesky_impl::ppotrs_bytes<T>(side, n, nrhs, false));
+    return std::max(fb, cholesky_impl::ppotrs_bytes<T>(side, n, nrhs, wide));
 }
 
 template <class T>
-void pposv_run_unstaged(const DdlaHandle_t& h, char side, char uplo, int n, int nrhs, T* A, const int* da, T* B,
-                        const int* db, int& info, void* backend_work, std::size_t backend_bytes)
+void pposv_exec(const DdlaHandle_t& h, char side, char uplo, int n, int nrhs, T* A, const int* da, T* B,
+                const int* db, int& info, void* backend_work, std::size_t backend_bytes, bool wide)
 {
     if (n == 0) {
         info = 0;
@@ -528,12 +521,12 @@ void pposv_run_unstaged(const DdlaHandle_t& h, char side, char uplo, int n, int 
     }
     cholesky_impl::ppotrf_run<T>(h, uplo, n, A, 1, 1, da, info, backend_work, backend_bytes, nullptr, 0);
     if (info == 0)
-        cholesky_impl::ppotrs_exec<T>(h, side, uplo, n, nrhs, A, da, B, db, backend_work, backend_bytes, false);
+        cholesky_impl::ppotrs_exec<T>(h, side, uplo, n, nrhs, A, da, B, db, backend_work, backend_bytes, wide);
 }
 
-template std::size_t pposv_unstaged_bytes<double>(char, int, int);
-template void pposv_run_unstaged<double>(const DdlaHandle_t&, char, char, int, int, double*, const int*, double*,
-                                         const int*, int&, void*, std::size_t);
+template std::size_t pposv_bytes<double>(char, int, int, bool);
+template void pposv_exec<double>(const DdlaHandle_t&, char, char, int, int, double*, const int*, double*, const int*,
+                                 int&, void*, std::size_t, bool);
 
 
 // ---------------------------------------------------------------------------

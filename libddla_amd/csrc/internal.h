@@ -167,14 +167,14 @@ template <class R>
 void diag_logdet(const DdlaHandle_t& h, int n, const std::complex<R>* A, int lda, std::complex<R>& result);
 } // namespace complex_impl
 
-// pposv with the 64-row sweeps whatever the order (no staged-solve work, so
-// the workspace stays at about 512 bytes per row): its backend bytes and its
-// run (ia = ja = ib = jb = 1, arguments already checked; cholesky.cpp).
+// pposv's backend bytes and its run (ia = ja = ib = jb = 1, arguments already
+// checked; cholesky.cpp).  wide: with the 128-row solve sweeps where pposv takes
+// them (1 KB of work per row in FP64), else with the 64-row ones (512 bytes).
 template <class T>
-std::size_t pposv_unstaged_bytes(char side, int n, int nrhs);
+std::size_t pposv_bytes(char side, int n, int nrhs, bool wide);
 template <class T>
-void pposv_run_unstaged(const DdlaHandle_t& h, char side, char uplo, int n, int nrhs, T* A, const int* descA, T* B,
-                        const int* descB, int& info, void* backend_work, std::size_t backend_bytes);
+void pposv_exec(const DdlaHandle_t& h, char side, char uplo, int n, int nrhs, T* A, const int* descA, T* B,
+                const int* descB, int& info, void* backend_work, std::size_t backend_bytes, bool wide);
 
 // FP64 pposv on the library's static device scratch (noalloc.cpp): no
 // hipMalloc / hipFree; throws std::invalid_argument when the call needs more

@@ -8,7 +8,7 @@
 #include "kernels.h"
 #include "gemm_tile.h"
 #include "solve_tile.h"
-#include "stage_tile.h"
+#include "wide_tile.h"
 #include "potf2_tile.h"
 #include "panel_host.h"
 #include "panel_tile.h"
@@ -851,103 +851,57 @@ void potrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long l
     check_launch("potrs");
 }
 
-bool stage_solve(int n, int nrhs) { return n >= kStageMinOrder && nrhs > 0 && !trsm_splits(n, nrhs); }
-
-namespace {
-// Layout of the staged solve's work: [E | M forward | M backward | accumulators | counters].
-struct StageLayout {
-    size_t e, mf, mb, acc, sync, total;
-};
-StageLayout stage_layout(int n, int nrhs, size_t elem)
+// From 640 rows (FP64), 448 (FP32) the 128-row sweeps are the faster ones.  A solve
+// with 64 right-hand sides, 64-row against 128-row sweeps with their preparation
+// and the return: FP64 n = 512: 127 / 137 us, 768: 169 / 160, 1024: 211 / 185;
+// FP32 n = 384: 89 / 93, 512: 104 / 100, 1024: 165 / 128.
+bool wide_solve(int n, int nrhs, size_t elem)
 {
-    using namespace stage_detail;
-    const size_t nst = (size_t)(n + kS - 1) / kS, slabs = (size_t)(nrhs + kSB - 1) / kSB;
-    const size_t nblk = (size_t)(n + kSB - 1) / kSB;
-    const size_t block = nst * kS * kS * elem;
-    StageLayout l{};
-    size_t off = 0;
-    auto put = [&](size_t bytes) {
-        const size_t at = off;
-        off += (bytes + 255) / 256 * 256;
-        return at;
-    };
-    l.e = put(block);
-    l.mf = put(block);
-    l.mb = put(block);
-    l.acc = put(slabs * (size_t)n * kSB * elem);
-    l.sync = put(slabs * (size_t)sync_ints((int)nst, (int)nblk) * sizeof(int));
-    l.total = off;
-    return l;
+    return n >= (elem == sizeof(double) ? 640 : 448) && nrhs > 0 && !trsm_splits(n, nrhs);
 }
 
-template <class T>
-stage_detail::StageArgs<T> stage_args(bool upper, int n, int nrhs, const T* L, long long ldl, const T* dinv, T* B,
-                                      long long ldb, void* work, int* error)
+namespace {
+size_t wide_inverse_bytes(int n, size_t elem)
 {
-    using namespace stage_detail;
-    const StageLayout l = stage_layout(n, nrhs, sizeof(T));
-    char* w = static_cast<char*>(work);
-    StageArgs<T> a{};
-    a.n = n;
-    a.nrhs = nrhs;
-    a.nst = (n + kS - 1) / kS;
-    a.nblk = (n + kSB - 1) / kSB;
-    a.L = L;
-    a.ldl = ldl;
-    a.upper = upper ? 1 : 0;
-    a.dinv = dinv;
-    a.E = reinterpret_cast<T*>(w + l.e);
-    a.M = reinterpret_cast<T*>(w + l.mf);
-    a.B = B;
-    a.ldb = ldb;
-    a.acc = reinterpret_cast<T*>(w + l.acc);
-    a.sync = reinterpret_cast<int*>(w + l.sync);
-    a.error = error;
-    a.spin_limit = wait_limit();
-    return a;
+    return ((size_t)wide_detail::blocks(n) * wide_detail::kWB * wide_detail::kWB * elem + 255) / 256 * 256;
 }
 } // namespace
 
-size_t stage_work_bytes(int n, int nrhs, size_t elem) { return stage_solve(n, nrhs) ? stage_layout(n, nrhs, elem).total : 0; }
-
-template <class T>
-void stage_prepare(hipStream_t s, bool upper, int n, const T* L, long long ldl, const T* dinv, void* work)
+size_t wide_work_bytes(int n, int nrhs, size_t elem)
 {
-    using namespace stage_detail;
-    StageArgs<T> a = stage_args<T>(upper, n, 1, L, ldl, dinv, nullptr, 0, work, nullptr);
-    const StageLayout l = stage_layout(n, 1, sizeof(T));
-    stage_inverse_kernel<T><<<dim3((unsigned)a.nst, kBlocks), kThreads, 0, s>>>(a);
-    check_launch("stage_prepare");
-    if (a.nst < 2) return;
-    const dim3 grid((unsigned)(a.nst - 1), kBlocks, kBlocks);
-    stage_product_kernel<T, false><<<grid, kThreads, 0, s>>>(a);
-    check_launch("stage_prepare");
-    a.M = reinterpret_cast<T*>(static_cast<char*>(work) + l.mb);
-    stage_product_kernel<T, true><<<grid, kThreads, 0, s>>>(a);
-    check_launch("stage_prepare");
+    if (!wide_solve(n, nrhs, elem)) return 0;
+    return wide_inverse_bytes(n, elem) + ((size_t)wide_detail::slabs(nrhs) * 4 * sizeof(int) + 255) / 256 * 256;
 }
 
 template <class T>
-void stage_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long long ldl, T* B, long long ldb,
-                  void* work, int* error)
+void wide_prepare(hipStream_t s, bool upper, int n, const T* L, long long ldl, void* work)
 {
-    using namespace stage_detail;
-    if (n <= 0 || nrhs <= 0) return;
-    if (!stage_solve(n, nrhs)) throw std::logic_error("stage_sweeps: order or right-hand sides out of range");
-    StageArgs<T> a = stage_args<T>(upper, n, nrhs, L, ldl, nullptr, B, ldb, work, error);
-    const StageLayout l = stage_layout(n, nrhs, sizeof(T));
-    const int slabs = (nrhs + kSB - 1) / kSB;
-    const int counters = slabs * sync_ints(a.nst, a.nblk);
-    const dim3 grid((unsigned)a.nblk, (unsigned)slabs);
-    solve_detail::zero_ints_kernel<<<(counters + 255) / 256, 256, 0, s>>>(a.sync, counters);
-    check_launch("stage_sweeps");
-    stage_sweep_kernel<T, false><<<grid, kThreads, 0, s>>>(a);
-    check_launch("stage_sweeps");
-    a.M = reinterpret_cast<T*>(static_cast<char*>(work) + l.mb);
-    solve_detail::zero_ints_kernel<<<(counters + 255) / 256, 256, 0, s>>>(a.sync, counters);
-    check_launch("stage_sweeps");
-    stage_sweep_kernel<T, true><<<grid, kThreads, 0, s>>>(a);
-    check_launch("stage_sweeps");
+    wide_detail::wide_inverse_kernel<T><<<wide_detail::blocks(n), 256, 0, s>>>(upper, n, L, ldl,
+                                                                               static_cast<T*>(work));
+    check_launch("wide_prepare");
+}
+
+template <class T>
+void wide_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long long ldl, T* B, long long ldb,
+                 void* work, int* error)
+{
+    using namespace wide_detail;
+    if (!wide_solve(n, nrhs, sizeof(T))) throw std::logic_error("wide_sweeps: order or right-hand sides out of range");
+    const int ns = slabs(nrhs);
+    int* sync = reinterpret_cast<int*>(static_cast<char*>(work) + wide_inverse_bytes(n, sizeof(T)));
+    const int vec = (uintptr_t)L % 16 == 0 && ldl % Mfma<T>::kVec == 0;
+    WideArgs<T> a{n, nrhs, blocks(n), ns, L, ldl, static_cast<const T*>(work), B, ldb, vec, sync, error,
+                  wait_limit()};
+    const unsigned grid = (unsigned)(a.nblk * ns);
+    zero_counters_kernel<<<1, 256, 0, s>>>(sync, 4 * ns);
+    check_launch("wide_sweeps");
+    if (upper) wide_sweep_kernel<T, false, false><<<grid, kWThreads, 0, s>>>(a);
+    else wide_sweep_kernel<T, false, true><<<grid, kWThreads, 0, s>>>(a);
+    check_launch("wide_sweeps");
+    a.sync += 2 * ns;
+    if (upper) wide_sweep_kernel<T, true, true><<<grid, kWThreads, 0, s>>>(a);
+    else wide_sweep_kernel<T, true, false><<<grid, kWThreads, 0, s>>>(a);
+    check_launch("wide_sweeps");
 }
 
 template <class T>
@@ -1315,8 +1269,8 @@ void convert(hipStream_t s, int m, int n, const S* in, long long ldi, D* out, lo
     template void potrs_sweeps<T>(hipStream_t, bool, int, int, const T*, long long, const T*, T*, long long,   \
                                   void*, int*);                                                               \
     template void add_diagonal<T>(hipStream_t, int, T*, long long, T);                                        \
-    template void stage_prepare<T>(hipStream_t, bool, int, const T*, long long, const T*, void*);                \
-    template void stage_sweeps<T>(hipStream_t, bool, int, int, const T*, long long, T*, long long, void*, int*);  \
+    template void wide_prepare<T>(hipStream_t, bool, int, const T*, long long, void*);                           \
+    template void wide_sweeps<T>(hipStream_t, bool, int, int, const T*, long long, T*, long long, void*, int*);  \
     template void trsm_sweep<T>(hipStream_t, bool, bool, int, int, const T*, long long, const T*, T*, long long, \
                                 void*, int*);                                                                 \
     template void trsm<T>(hipStream_t, bool, bool, int, int, const T*, long long, const T*, T*, long long,       \

@@ -61,16 +61,18 @@ void pposv_noalloc(const DdlaHandle_t& h, char side, char uplo, char trans, int 
         info = 0;
         return;
     }
-    // The 64-row sweeps keep the workspace at about 512 bytes per row; the
-    // staged solve's prepared blocks (12 KB per row in FP64) would not fit.
-    const std::size_t bytes = pposv_unstaged_bytes<double>(side, n, nrhs);
+    // pposv's own sweeps where their work fits (1 KB per row), else the 64-row
+    // ones (512 bytes per row)
+    std::size_t bytes = pposv_bytes<double>(side, n, nrhs, true);
+    const bool wide = bytes <= kNoAllocScratchBytes;
+    if (!wide) bytes = pposv_bytes<double>(side, n, nrhs, false);
     if (bytes > kNoAllocScratchBytes)
         throw std::invalid_argument("pposv_noalloc: this order and right-hand-side count need " +
                                     std::to_string(bytes) + " bytes of scratch, more than the " +
                                     std::to_string(kNoAllocScratchBytes) +
                                     " bytes of the static scratch (use pposv, which allocates)");
     void* work = scratch_address(h->device);
-    pposv_run_unstaged<double>(h, side, uplo, n, nrhs, A, descA, B, descB, info, work, bytes);
+    pposv_exec<double>(h, side, uplo, n, nrhs, A, descA, B, descB, info, work, bytes, wide);
     DDLA_HIP(hipStreamSynchronize(h->stream));
 }
 

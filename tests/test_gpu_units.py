@@ -1,11 +1,13 @@
-"""Factorizations at the edges of their blocks: orders around the 64-row blocks
-and the largest one-panel order (4096), the same matrix by narrow panels, and complex
-elements.
+"""Factorizations and solves at the edges of their blocks: orders around the
+64-row blocks and the largest one-panel order (4096), the same matrix by narrow
+panels, complex elements, and the 128-row solve sweeps over orders, right-hand
+sides, triangles and sides.
 
-Checked against the problem itself, in float64 on the GPU.  Tolerance: a
+Checked against the problem itself, in float64 on the GPU.  Tolerances: a
 backward-stable factorization has |A - L L^H|_F <= c n eps |A|_F with c a small
 constant times the condition of the inverted 64 x 64 diagonal blocks (below 5
-here: every spectrum lies in [0.5, 4.6]), so 10 n eps."""
+here: every spectrum lies in [0.5, 4.6]), so 10 n eps; a solve with inverted 128 x
+128 blocks has the residual bound 10 n eps |A|_F |X|_F likewise."""
 import numpy as np
 import pytest
 
@@ -65,3 +67,28 @@ def test_factor_units(handle, dtype, n, uplo):
         finally:
             dd.lib.ddla_c_set_panel_width(previous)
         assert residual(a, s2, uplo) <= tol
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128])
+@pytest.mark.parametrize("n,nrhs", [(1, 1), (129, 17), (447, 3), (448, 1), (513, 16), (639, 33), (640, 15), (641, 17),
+                                    (767, 64), (1000, 255)])
+@pytest.mark.parametrize("uplo,side", [("L", "L"), ("U", "L"), ("L", "R")])
+def test_solve_sweeps(handle, dtype, n, nrhs, uplo, side):
+    import torch
+
+    print(f"case sweeps n={n} nrhs={nrhs} {np.dtype(dtype).name} {uplo} {side}", flush=True)
+    a, gen = system(n, dtype, 7 * n + nrhs)
+    A, _ = factor(handle, a, dtype, uplo)
+    rows, cols = (n, nrhs) if side == "L" else (nrhs, n)
+    pad = 5  # rows of B's parent that stay as they are
+    full = torch.randn(cols, rows + pad, dtype=a.dtype, device="cuda", generator=gen)
+    b = full.to(getattr(torch, TORCH[dtype])).clone()
+    keep = b.clone()
+    torch.cuda.synchronize()
+    B = dd.DistributedMatrix.from_torch(handle, b, rows, cols)
+    dd.ppotrs(A, B, uplo, side)
+    x, b0 = b[:, :rows].t().to(a.dtype).contiguous(), keep[:, :rows].t().to(a.dtype).contiguous()
+    r = b0 - (torch.mm(a, x) if side == "L" else torch.mm(x, a))
+    norm = torch.linalg.norm
+    assert (norm(r) / (norm(a) * norm(x))).item() <= 10 * n * np.finfo(dtype).eps
+    assert torch.equal(b[:, rows:], keep[:, rows:])
