@@ -13,10 +13,14 @@
 //     identity) in the accumulator layout, in which the four columns of a step
 //     are one register and, as they stand, both operands of the 16x16x4
 //     product that applies them to the later columns.  The step's 4 x 4
-//     diagonal block is factored and inverted by every lane redundantly, so
-//     neither a pivot's chain to the next one nor the strip has any exchange
-//     between wavefronts in it, and the pass turns the identity into
-//     L(b, b)^-T, the inverse of the strip's diagonal block;
+//     diagonal block is factored by every lane redundantly, and every lane
+//     finishes the four columns of its row by substitution, so neither a pivot's
+//     chain to the next one nor the strip has any exchange between wavefronts in
+//     it, and the pass turns the identity into L(b, b)^-T, the inverse of the
+//     strip's diagonal block (multiplied by an explicit inverse of the 4 x 4
+//     block instead, at the same speed, the columns of a nearly singular one were
+//     off by 47 n eps instead of 0.5, pivots among them down to negative ones in
+//     a factor reported complete, and a NaN pivot reached the columns before it);
 //   * between two passes the strip is applied to the next strip's columns
 //     (update_tile), and to the columns beyond while the next pass runs; the
 //     wavefronts that have no rows left in a strip also form, during the
@@ -92,13 +96,37 @@ __device__ __forceinline__ double masked(double x, int mask)
 
 __device__ __forceinline__ float masked(float x, int mask) { return __int_as_float(__float_as_int(x) & mask); }
 
-// The bits of x and y together (one of them masked to zero).
-__device__ __forceinline__ double merged(double x, double y)
+// x[c] = the v of lane 16 c + l % 16, for every lane l.
+__device__ __forceinline__ void gather_columns(unsigned v, unsigned (&x)[4])
 {
-    return __longlong_as_double(__double_as_longlong(x) | __double_as_longlong(y));
+    // odd rows of sixteen lanes of the first operand against even ones of the second, then the halves likewise
+    const auto pairs = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    const auto even = __builtin_amdgcn_permlane32_swap(pairs[0], pairs[0], false, false);
+    const auto odd = __builtin_amdgcn_permlane32_swap(pairs[1], pairs[1], false, false);
+    x[0] = even[0];
+    x[1] = odd[0];
+    x[2] = even[1];
+    x[3] = odd[1];
 }
 
-__device__ __forceinline__ float merged(float x, float y) { return __int_as_float(__float_as_int(x) | __float_as_int(y)); }
+__device__ __forceinline__ void gather_columns(float v, float (&x)[4])
+{
+    unsigned u[4];
+    gather_columns(__float_as_uint(v), u);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) x[c] = __uint_as_float(u[c]);
+}
+
+__device__ __forceinline__ void gather_columns(double v, double (&x)[4])
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    unsigned lo[4], hi[4];
+    gather_columns((unsigned)b, lo);
+    gather_columns((unsigned)(b >> 32), hi);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        x[c] = __longlong_as_double((long long)(((unsigned long long)hi[c] << 32) | lo[c]));
+}
 
 // 1 / sqrt(d) for d > 0: the hardware estimate and one third-order step (FP64:
 // with e = 1 - d y^2, y (1 + e/2 + 3 e^2 / 8); the estimate's ~2^-23 becomes
@@ -157,8 +185,6 @@ __device__ __forceinline__ int factor_strip(real_t<T>* S, real_t<T>* X,
             x[p][r] = wave == 0 ? (p == 0 && li == c ? R(1) : R(0))
                                 : S[p * kPlane + (r0 + c) * kL + r0 + kW * wave + li];
         }
-    auto unit = [&](int k) { return element<T>(g == k ? R(1) : R(0), R(0)); };
-    const T u1 = unit(1), u2 = unit(2), u3 = unit(3);
     R below[4][P];               // the finished columns of x
     unsigned long long bad = 0;  // bit j: the pivot of column j is not positive
     auto check = [&](R v, int j) { bad |= __ballot(!(v > R(0))) & (1ull << j); };
@@ -182,33 +208,28 @@ __device__ __forceinline__ int factor_strip(real_t<T>* S, real_t<T>* X,
         check(d1, 4 * q + 1);
         check(d2, 4 * q + 2);
         check(d3, 4 * q + 3);
-        // column g of the 4 x 4 inverse, then its row diag_row(l % 16) as the left operand
-        const T e0 = scale(unit(0), y0), e1 = scale(sub_mul(u1, l10, e0), y1);
-        const T e2 = scale(sub_mul(sub_mul(u2, l20, e0), l21, e1), y2);
-        const T e3 = scale(sub_mul(sub_mul(sub_mul(u3, l30, e0), l31, e1), l32, e2), y3);
-        R inv[P], next[P], own[P];
+        // the four finished columns of every row, W = A L44^-H by substitution: a lane
+        // takes the step's elements of its row from the four lanes that hold them
+        auto substitute = [&](const tile_acc<T>& block, R (&column)[P]) __attribute__((always_inline)) {
+            R v[P][4];
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            inv[p] = merged(merged(masked(plane(e0, p), -(int)(pr == 0)), masked(plane(e1, p), -(int)(pr == 1))),
-                            merged(masked(plane(e2, p), -(int)(pr == 2)), masked(plane(e3, p), -(int)(pr == 3))));
-            own[p] = d[p][q];
-        }
-        // the four finished columns W = A L44^-H, transposed: conj(inv) times the register
-        tile_acc<T> w;
-        clear<T>(w);
-        mma_conj_add(inv, own, w);
+            for (int p = 0; p < P; ++p) gather_columns(block[p][q], v[p]);
+            auto at = [&](int c) { return element<T>(v[0][c], v[P - 1][c]); };
+            const T w0 = scale(at(0), y0);
+            const T w1 = scale(sub_mul_conj(at(1), w0, l10), y1);
+            const T w2 = scale(sub_mul_conj(sub_mul_conj(at(2), w0, l20), w1, l21), y2);
+            const T w3 = scale(sub_mul_conj(sub_mul_conj(sub_mul_conj(at(3), w0, l30), w1, l31), w2, l32), y3);
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            diag[q][p] = w[p][0];
-            next[p] = masked(-w[p][0], -(int)(pr >= 4 * q + 4));  // the rows that later columns multiply
-        }
+            for (int p = 0; p < P; ++p)
+                column[p] = g < 2 ? (g == 0 ? plane(w0, p) : plane(w1, p)) : (g == 2 ? plane(w2, p) : plane(w3, p));
+        };
+        R next[P];
+        substitute(d, diag[q]);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            next[p] = masked(-diag[q][p], -(int)(pr >= 4 * q + 4));  // the rows that later columns multiply
         if (q < 3) mma_conj_add(next, diag[q], d);
-#pragma unroll
-        for (int p = 0; p < P; ++p) own[p] = x[p][q];
-        clear<T>(w);
-        mma_conj_add(inv, own, w);
-#pragma unroll
-        for (int p = 0; p < P; ++p) below[q][p] = w[p][0];
+        substitute(x, below[q]);
         if (q < 3) mma_conj_add(next, below[q], x);
     }
 #pragma unroll
