@@ -93,3 +93,29 @@ def test_failed_row_keeps_its_finished_columns(handle, dtype):
             if np.isnan(value):
                 assert info == p + 1
             assert np.abs(A.to_global_matrix()[p, :p] - ref[p, :p]).max() <= tol, (p, value)
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_complex_block_rounds_once_a_step(handle, dtype):
+    """Order 64, well conditioned: the mean relative error of the factor.  Elements round
+    at the scale of the trailing matrix (about half of A's) once per four columns: 16
+    roundings of independent sign and rms u / sqrt(3) make 16^(1/2) / (2 sqrt(3)) = 1.2 u,
+    the strip products' and the last operations' own roundings less than that again.
+    Rounding at each of the 128 real terms would make 3.3 u; allowed are 2 u = eps."""
+    print(f"case complex block rounding {np.dtype(dtype).name}", flush=True)
+    rng = np.random.RandomState(13)
+    n, errors = 64, []
+    for _ in range(12):
+        a = nearly_singular(dtype, n, n, 0, rng) / n + np.eye(n, dtype=dtype)
+        a = ((a + a.conj().T) / 2).astype(dtype)
+        # column by column in extended precision
+        wide = a.astype(np.clongdouble)
+        ref = np.zeros_like(wide)
+        for j in range(n):
+            ref[j, j] = np.sqrt((wide[j, j] - (ref[j, :j] * ref[j, :j].conj()).sum()).real)
+            ref[j + 1:, j] = (wide[j + 1:, j] - ref[j + 1:, :j] @ ref[j, :j].conj()) / ref[j, j]
+        A = dd.DistributedMatrix.from_global_matrix(handle, a)
+        assert dd.ppotrf(A, "L")[1] == 0
+        low = np.tril(A.to_global_matrix())
+        errors.append(float(np.sqrt((np.abs(low - ref) ** 2).sum() / (np.abs(ref) ** 2).sum())))
+    assert np.mean(errors) <= np.finfo(dtype).eps, np.mean(errors) / np.finfo(dtype).eps
