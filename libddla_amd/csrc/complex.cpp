@@ -11,7 +11,8 @@
 //   vbatched include/ddla/ddla.h:1878-1960 (mixed overloads: 'C' on a real operand is 'T')
 // The arithmetic is this project's: the real types' blocked factorization with
 // its two-panel look-ahead (potrf_blocked) on complex panels and the complex
-// GEMM tile, and one persistent launch per solve sweep (zsolve_tile.h).
+// GEMM tile, and one persistent launch per solve sweep (zsolve_tile.h), or for
+// many columns products of 64-row steps (solve_by_products).
 #include "internal.h"
 #include "kernels.h"
 #include "zkernels.h"
@@ -35,6 +36,43 @@ constexpr int kZB = 64;
 std::size_t zdiag_inverse_elems(int n) { return (std::size_t)((n + kZB - 1) / kZB) * kZB * kZB; }
 
 } // namespace
+
+// Solves A X = B in place (B n x nrhs) with A = L L^H given by its L view
+// (lower: L = A's lower triangle; upper: L = U^H of A's upper triangle) and the
+// inverses D_t of its 64 x 64 diagonal blocks: forward L Y = B, then backward
+// L^H X = Y, 64 rows a step (X_t = D_t B_t, then one product for all rows left).
+template <class R>
+void solve_by_products(DdlaStream* h, bool upper, int n, int nrhs, const std::complex<R>* A, long long lda,
+                       const std::complex<R>* dinv, std::complex<R>* B, long long ldb)
+{
+    using C = std::complex<R>;
+    const int nb = (n + kZB - 1) / kZB;
+    // B(rows) -= op(block (r0, c0) of the L view, m x k or k x m) B(at)
+    auto subtract = [&](int r0, int c0, char op, int m, int k, int rows, int at) {
+        if (m <= 0) return;
+        // upper: L(r, c) = conj(A(c, r)), so the block is stored conjugate transposed
+        const C* p = upper ? A + c0 + r0 * lda : A + r0 + c0 * lda;
+        const char stored = upper ? (op == 'N' ? 'C' : 'N') : op;
+        kern::zgemm<R>(h->stream, true, true, stored, 'N', m, nrhs, k, C(-1), p, lda, B + at, ldb, C(1), B + rows, ldb);
+    };
+    // B_t := D_t B_t, or D_t^H B_t: one row of tiles, each of which reads its columns before it writes them
+    auto multiply = [&](int t, char op) {
+        const int w = std::min(kZB, n - t * kZB);
+        C* bt = B + t * kZB;
+        kern::zgemm<R>(h->stream, true, true, op, 'N', w, nrhs, w, C(1), dinv + (long long)t * kZB * kZB, kZB, bt, ldb,
+                       C(0), bt, ldb);
+    };
+    for (int t = 0; t < nb; ++t) {
+        const int r0 = t * kZB, r1 = std::min(n, r0 + kZB);
+        multiply(t, 'N');
+        subtract(r1, r0, 'N', n - r1, r1 - r0, r1, r0);
+    }
+    for (int t = nb - 1; t >= 0; --t) {
+        const int r0 = t * kZB, r1 = std::min(n, r0 + kZB);
+        multiply(t, 'C');
+        subtract(r0, 0, 'C', r0, r1 - r0, 0, r0);
+    }
+}
 
 template <class R>
 std::size_t ppotrs_bytes(char side, int n, int nrhs)
@@ -94,7 +132,10 @@ void ppotrs_run(const DdlaHandle_t& h, char side, char uplo, int n, int nrhs, co
     fill_int(h->stream, error, 0);
     auto sweeps = [&](C* b, long long ld) {
         LaunchTimer timer(h, kClassSolve, 8.0 * n * (double)n * nrhs, 2.0 * n * n * sizeof(R));
-        kern::zpotrs_sweeps<R>(h->stream, upper, n, nrhs, A, lda, dinv, b, ld, sync, error);
+        if (kern::zsolve_sweeps<R>(n, nrhs))
+            kern::zpotrs_sweeps<R>(h->stream, upper, n, nrhs, A, lda, dinv, b, ld, sync, error);
+        else
+            solve_by_products<R>(h, upper, n, nrhs, A, lda, dinv, b, ld);
     };
     {
         LaunchTimer timer(h, kClassTrtri, 4.0 * n * kZB * kZB / 3.0);

@@ -41,6 +41,10 @@ template <class R>
 void ztrtri_diag_blocks(hipStream_t s, bool upper, int n, const std::complex<R>* A, long long lda,
                         std::complex<R>* inv);
 
+// Whether zpotrs_sweeps is the faster way to solve (zkernels.hip).
+template <class R>
+bool zsolve_sweeps(int n, int nrhs);
+
 // L Y = B, then L^H X = Y in place on B (n x nrhs) with the L view of A and its
 // inverted diagonal blocks dinv (ztrtri_diag_blocks): one persistent launch per
 // sweep.  sync: zsolve_sync_bytes(nrhs) bytes; *error is set to 1 if a wait

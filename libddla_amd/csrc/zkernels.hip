@@ -533,6 +533,19 @@ std::size_t zsolve_sync_bytes(int nrhs)
     return ((std::size_t)zsolve_detail::slabs(nrhs) * 4 * sizeof(int) + 255) / 256 * 256;
 }
 
+// The sweeps are bound by the chain of blocks while their workgroups (64-row blocks
+// times 16-column slabs) are a few waves of the chip, and by reading the factor once a
+// slab beyond; products of 64-row steps read it once for all columns.  A solve by
+// products / by sweeps, us: complex128 n = 1500 with 768 columns (1152 workgroups)
+// 2174 / 2033, n = 600 with 2048 (1280) 906 / 960, n = 4000 with 1024 (4032) 8036 /
+// 17394; complex64 n = 1000 with 2048 (2048) 1011 / 1005, n = 600 with 4096 (2560)
+// 658 / 808, n = 4000 with 1024 (4032) 4699 / 7753.
+template <class R>
+bool zsolve_sweeps(int n, int nrhs)
+{
+    return (long long)((n + 63) / 64) * zsolve_detail::slabs(nrhs) <= (sizeof(R) == 8 ? 1200 : 2048);
+}
+
 template <class R>
 void zpotrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const std::complex<R>* A, long long lda,
                    const std::complex<R>* dinv, std::complex<R>* B, long long ldb, void* sync, int* error)
@@ -540,7 +553,6 @@ void zpotrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const std::comple
     using namespace zsolve_detail;
     if (n <= 0 || nrhs <= 0) return;
     const int ns = slabs(nrhs);
-    if (ns > 65535) throw std::invalid_argument("zpotrs_sweeps: too many right-hand sides");
     SweepArgs<R> a{n, nrhs, (n + kSB - 1) / kSB, reinterpret_cast<const Cx<R>*>(A), lda, upper ? 1 : 0,
                    reinterpret_cast<const Cx<R>*>(dinv), reinterpret_cast<Cx<R>*>(B), ldb, static_cast<int*>(sync),
                    error, wait_limit()};
@@ -597,6 +609,7 @@ void zdiag_logdet(hipStream_t s, int n, const std::complex<R>* A, long long lda,
                                     std::complex<R>, const void* const*, const int*, const void* const*,         \
                                     const int*, std::complex<R>, std::complex<R>* const*, const int*, int, int,  \
                                     int);                                                                        \
+    template bool zsolve_sweeps<R>(int, int);                                                                    \
     template void zpotrs_sweeps<R>(hipStream_t, bool, int, int, const std::complex<R>*, long long,               \
                                    const std::complex<R>*, std::complex<R>*, long long, void*, int*);            \
     template size_t panel_work_bytes<std::complex<R>>(int);                                                      \

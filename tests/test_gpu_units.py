@@ -92,3 +92,34 @@ def test_solve_sweeps(handle, dtype, n, nrhs, uplo, side):
     norm = torch.linalg.norm
     assert (norm(r) / (norm(a) * norm(x))).item() <= 10 * n * np.finfo(dtype).eps
     assert torch.equal(b[:, rows:], keep[:, rows:])
+
+
+def column_error(a, x, b):
+    """max over columns of |b - a x| / (|a| |x|) in infinity norms, float64 / complex128 on the GPU."""
+    import torch
+
+    r = (b - torch.mm(a, x)).abs().amax(0)
+    return (r / (a.abs().sum(1).max() * x.abs().amax(0))).max().item()
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n,nrhs", [(3, 1048577), (129, 6416), (129, 11008), (700, 3000)])
+@pytest.mark.parametrize("uplo,side", [("L", "L"), ("U", "L"), ("L", "R"), ("U", "R")])
+def test_complex_solves_with_many_columns(handle, dtype, n, nrhs, uplo, side):
+    """On both sides of the change from sweeps to products, and more columns than one launch's grid
+    takes in its second dimension.  Column by column, within the suite's 0.05 n eps (n >= 64)."""
+    import torch
+
+    print(f"case many columns n={n} nrhs={nrhs} {np.dtype(dtype).name} {uplo} {side}", flush=True)
+    a, gen = system(n, dtype, 5 * n)
+    A, _ = factor(handle, a, dtype, uplo)
+    rows, cols = (n, nrhs) if side == "L" else (nrhs, n)
+    b0 = torch.randn(cols, rows, dtype=a.dtype, device="cuda", generator=gen).to(getattr(torch, TORCH[dtype]))
+    b = b0.clone()
+    torch.cuda.synchronize()
+    B = dd.DistributedMatrix.from_torch(handle, b, rows, cols)
+    dd.ppotrs(A, B, uplo, side)
+    x, c = b.t().to(a.dtype).contiguous(), b0.t().to(a.dtype).contiguous()
+    if side == "R":  # X A = C  is  A X^H = C^H
+        x, c = x.mH.contiguous(), c.mH.contiguous()
+    assert column_error(a, x, c) <= 0.05 * max(n, 64) * np.finfo(dtype).eps
