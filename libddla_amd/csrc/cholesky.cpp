@@ -388,11 +388,9 @@ std::size_t ppotrs_bytes(char side, int n, int nrhs, bool wide)
     if (n == 0 || nrhs == 0) return 0;
     // [ error word | wide solve's work, or: inverses of the 64 x 64 diagonal blocks | sweep counters |
     //   transposed B (side 'R') ]
-    std::size_t b = detail::padded_bytes<int>(1);
-    if (wide && kern::wide_solve(n, nrhs, sizeof(T)))
-        b += detail::padded_bytes<char>(kern::wide_work_bytes(n, nrhs, sizeof(T)));
-    else
-        b += detail::padded_bytes<T>(diag_inverse_elems(n)) + kern::solve_work_bytes(nrhs);
+    std::size_t b = detail::padded_bytes<T>(diag_inverse_elems(n)) + kern::solve_work_bytes(nrhs);
+    if (wide) b = std::max(b, detail::padded_bytes<char>(kern::wide_work_bytes(n, nrhs, sizeof(T))));  // for either uplo
+    b += detail::padded_bytes<int>(1);
     if (side == 'R') b += detail::padded_bytes<T>((std::size_t)n * nrhs);
     return b;
 }
@@ -419,7 +417,7 @@ void ppotrs_exec(const DdlaHandle_t& h, char side, char uplo, int n, int nrhs, c
     char* w = static_cast<char*>(backend_work);
     int* error = detail::take<int>(w, 1);
     fill_int(h->stream, error, 0);
-    wide = wide && kern::wide_solve(n, nrhs, sizeof(T));
+    wide = wide && kern::wide_solve(upper, n, nrhs, sizeof(T));
     void* wide_work = nullptr;
     T* dinv = nullptr;
     void* sync = nullptr;

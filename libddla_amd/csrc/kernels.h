@@ -129,12 +129,12 @@ void potrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long l
                   long long ldb, void* work, int* error);
 
 // The solves with a kept factor over 128-row blocks and 16-column slabs
-// (wide_tile.h), for right-hand sides below kTrsmMinColumns or orders that trsm
-// does not split (wide_solve).  wide_prepare forms, once per factor, the inverses
-// of its 128 x 128 diagonal blocks in work (wide_work_bytes(n, nrhs, sizeof(T))
-// bytes); wide_sweeps then solves L Y = B and L^T X = Y in place on B (n x nrhs),
-// any number of times; *error as for potrs_sweeps.
-bool wide_solve(int n, int nrhs, size_t elem);
+// (wide_tile.h), where they are the faster ones (wide_solve).  wide_prepare forms,
+// once per factor, the inverses of its 128 x 128 diagonal blocks in work
+// (wide_work_bytes(n, nrhs, sizeof(T)) bytes, for either triangle); wide_sweeps
+// then solves L Y = B and L^T X = Y in place on B (n x nrhs), any number of
+// times; *error as for potrs_sweeps.
+bool wide_solve(bool upper, int n, int nrhs, size_t elem);
 size_t wide_work_bytes(int n, int nrhs, size_t elem);
 template <class T>
 void wide_prepare(hipStream_t s, bool upper, int n, const T* L, long long ldl, void* work);

@@ -851,13 +851,26 @@ void potrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long l
     check_launch("potrs");
 }
 
-// From 640 rows (FP64), 448 (FP32) the 128-row sweeps are the faster ones.  A solve
-// with 64 right-hand sides, 64-row against 128-row sweeps with their preparation
-// and the return: FP64 n = 512: 127 / 137 us, 768: 169 / 160, 1024: 211 / 185;
-// FP32 n = 384: 89 / 93, 512: 104 / 100, 1024: 165 / 128.
-bool wide_solve(int n, int nrhs, size_t elem)
+// From 640 rows (FP64), 448 (FP32) of a lower factor the 128-row sweeps are the faster
+// ones; an upper one, whose forward sweep reads along rows, pays from 896 / 768, and
+// from 640 with 64 columns.  64-row against 128-row sweeps with their preparation and
+// the return, us: FP64 lower, 64 columns, n = 512: 127 / 137, 640: 165 / 149, 1024: 211
+// / 185; upper, 1 column, n = 704: 159 / 170, 896: 191 / 186; FP32 lower, 64 columns, n
+// = 384: 89 / 93, 512: 104 / 100, 1024: 165 / 128; upper, 1 column, n = 640: 122 / 125,
+// 768: 137 / 131.
+// With 256 columns and more (n <= 1024 then) the 128-row sweeps' chains have to run side
+// by side, one workgroup a CU: FP64 lower n = 1024, 512 columns (256 workgroups) 255 /
+// 196, 768 (384) 251 / 258; FP32 upper, 512 columns 194 / 159, 768 197 / 199.  In FP32
+// with a lower factor they stay ahead from 512 rows on up to eight times as many: n =
+// 512, 2048 columns (512) 149 / 137, n = 1024 (1024) 312 / 281; n = 800, 8192 (3584) 673
+// / 703.
+bool wide_solve(bool upper, int n, int nrhs, size_t elem)
 {
-    return n >= (elem == sizeof(double) ? 640 : 448) && nrhs > 0 && !trsm_splits(n, nrhs);
+    const bool wide_type = elem == sizeof(double);
+    const int from = !upper ? (wide_type ? 640 : 448) : nrhs >= 64 ? 640 : wide_type ? 896 : 768;
+    if (n < from || nrhs <= 0 || trsm_splits(n, nrhs)) return false;
+    const long long workgroups = (long long)wide_detail::blocks(n) * wide_detail::slabs(nrhs);
+    return nrhs < kTrsmMinColumns || workgroups <= (!wide_type && !upper && n >= 512 ? 2048 : 256);
 }
 
 namespace {
@@ -869,7 +882,7 @@ size_t wide_inverse_bytes(int n, size_t elem)
 
 size_t wide_work_bytes(int n, int nrhs, size_t elem)
 {
-    if (!wide_solve(n, nrhs, elem)) return 0;
+    if (!wide_solve(false, n, nrhs, elem)) return 0;  // an upper factor takes no others
     return wide_inverse_bytes(n, elem) + ((size_t)wide_detail::slabs(nrhs) * 4 * sizeof(int) + 255) / 256 * 256;
 }
 
@@ -886,7 +899,7 @@ void wide_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long lo
                  void* work, int* error)
 {
     using namespace wide_detail;
-    if (!wide_solve(n, nrhs, sizeof(T))) throw std::logic_error("wide_sweeps: order or right-hand sides out of range");
+    if (!wide_solve(upper, n, nrhs, sizeof(T))) throw std::logic_error("wide_sweeps: order or right-hand sides out of range");
     const int ns = slabs(nrhs);
     int* sync = reinterpret_cast<int*>(static_cast<char*>(work) + wide_inverse_bytes(n, sizeof(T)));
     const int vec = (uintptr_t)L % 16 == 0 && ldl % Mfma<T>::kVec == 0;

@@ -142,7 +142,7 @@ void pposv_mixed_run(const DdlaHandle_t& h, char uplo, int n, int nrhs, T* A, co
         fill_int(s, error, 0);
         // every correction solves with the same factor: its diagonal blocks are
         // inverted once
-        const bool wide = kern::wide_solve(n, nrhs, sizeof(float));
+        const bool wide = kern::wide_solve(upper, n, nrhs, sizeof(float));
         if (wide) {
             LaunchTimer timer(h, kClassTrtri, (double)n * 128 * 128 / 3.0);
             kern::wide_prepare<float>(s, upper, n, a32, n, base + l.wide);

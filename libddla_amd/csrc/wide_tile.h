@@ -161,8 +161,9 @@ __global__ void zero_counters_kernel(int* p, int count)
 
 // Grid: nslab * nblk workgroups, slabs fastest, so that all slabs advance together.
 // DIRECT: Op(t, q)'s rows run along a stored column, else along a stored row
-// (BACKWARD == upper; with both in one kernel FP64's forward sweep spilled: 400 us
-// where it takes 370, n = 8192).
+// (BACKWARD == upper; with both in one kernel FP64's forward sweep spilled with a lower
+// factor too: 400 us where it takes 370, n = 8192.  With an upper one it still keeps 20
+// registers in memory).
 template <class T, bool BACKWARD, bool DIRECT>
 __global__ __launch_bounds__(kWThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void wide_sweep_kernel(
     WideArgs<T> a)

@@ -123,3 +123,22 @@ def test_complex_solves_with_many_columns(handle, dtype, n, nrhs, uplo, side):
     if side == "R":  # X A = C  is  A X^H = C^H
         x, c = x.mH.contiguous(), c.mH.contiguous()
     assert column_error(a, x, c) <= 0.05 * max(n, 64) * np.finfo(dtype).eps
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,nrhs,uplo", [(512, 1500, "L"), (800, 4700, "L"), (640, 816, "L"), (640, 817, "L"), (1024, 513, "L"),
+                                         (640, 64, "U"), (700, 63, "U"), (768, 1, "U"), (895, 2, "U"), (896, 2, "U"),
+                                         (1024, 512, "U"), (1024, 528, "U")])
+def test_solve_routes(handle, dtype, n, nrhs, uplo):
+    """Both sides of each line between the 64-row and the 128-row sweeps; column by column."""
+    import torch
+
+    print(f"case routes n={n} nrhs={nrhs} {np.dtype(dtype).name} {uplo}", flush=True)
+    a, gen = system(n, dtype, 3 * n + nrhs)
+    A, _ = factor(handle, a, dtype, uplo)
+    b0 = torch.randn(nrhs, n, dtype=a.dtype, device="cuda", generator=gen).to(getattr(torch, TORCH[dtype]))
+    b = b0.clone()
+    torch.cuda.synchronize()
+    dd.ppotrs(A, dd.DistributedMatrix.from_torch(handle, b, n, nrhs), uplo)
+    x, c = b.t().to(a.dtype).contiguous(), b0.t().to(a.dtype).contiguous()
+    assert column_error(a, x, c) <= 0.05 * n * np.finfo(dtype).eps
