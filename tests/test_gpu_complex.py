@@ -334,6 +334,16 @@ def test_complex_vbatched_ops(handle, dtype, ta, tb):
     run_vbatched(handle, dtype, ta, tb, SIZES, 0.75 - 1.25j, 0.5 + 0.25j)
 
 
+# the halves of a 64 x 64 tile (a wavefront each has none, one or all of its rows and columns), slab edges
+EDGES = [(m, n, k) for m in (1, 31, 33, 64, 65) for n in (16, 32, 49, 97) for k in (1, 15, 17, 64, 70)]
+
+
+@pytest.mark.parametrize("dtype", CTYPES)
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "C"), ("C", "T")])
+def test_complex_vbatched_tile_edges(handle, dtype, ta, tb):
+    run_vbatched(handle, dtype, ta, tb, EDGES, 0.75 - 1.25j, 0.5 + 0.25j)
+
+
 @pytest.mark.parametrize("dtype", CTYPES)
 def test_complex_vbatched_special_cases(handle, dtype):
     run_vbatched(handle, dtype, "C", "N", SIZES, 1.0j, 0.0, beta_zero_nan=True, pad=3)
