@@ -641,7 +641,7 @@ def main():
         solve_phase = {"ms_per_step": round(solve_ms, 3), "algorithmic_bytes": 8.0 * n * n,
                        "hbm_gb_s": round(8.0 * n * n / (solve_ms * 1e-3) / 1e9, 1), "peak_gb_s": 8000.0,
                        "frac": round(8.0 * n * n / (solve_ms * 1e-3) / 8e12, 4),
-                       "bound": "the 64-row-block dependency chain (latency), not HBM"}
+                       "bound": "the 128-row-block dependency chain (latency), not HBM"}
     traffic = None
     tfile = os.path.join(ROOT, "profiles", "trailing_update_traffic.json")
     if os.path.exists(tfile):
@@ -662,7 +662,7 @@ def main():
         "dtype": "f64",
         "data": "synthetic (Philox4x64-10 normals, seed 1; A = G G^T/n + 0.1 I)",
         "config": {"workload": f"FP64 pposv n={n} nrhs={nrhs} uplo={args.uplo}, A = G G^T/n + 0.1 I", "n": n,
-                   "nrhs": nrhs, "nb": 512, "panel_width": 768 if n >= 16384 else 512, "uplo": args.uplo},
+                   "nrhs": nrhs, "nb": 512, "panel_width": 768 if n >= 16384 else 512 if n > 4096 else n, "uplo": args.uplo},
         "pct_fp64_peak": round(100 * value / FP64_PEAK, 2),
         "backward_error": bwd,
         "roofline": {"bound": "mfma", "kernel": "trailing_update (FP64 MFMA syrk)", "achieved": round(achieved, 3),

@@ -46,8 +46,7 @@ constexpr int kIB = 64;  // diagonal block of potf2 and of the solves
 //   ms with 512 / 768 / 1024, while at n = 8192 512 is best.
 // * A batch of problems fills the chip with 512-column panels, which leave more
 //   of the work to the trailing updates; the split-product path keeps 512 (its
-//   panel buffers hold 512 columns).  With the launch profiler on, whose classes
-//   are the steps of the panel schedule, small orders take 512 too.
+//   panel buffers hold 512 columns).
 // A process-wide override (set_panel_width; 0 = the rule above) lets tests
 // run narrower and the 768-column panels at small orders.
 std::atomic<int> g_panel_width{0};
@@ -246,7 +245,7 @@ void potrf_blocked(DdlaStream* h, bool upper, int n, T* A, long long lda, int* i
         return;
     }
     const LView<T> v{A, lda};
-    const int NB = outer_block<T>(n, split != nullptr, batch.count == 1 && !h->profiling);
+    const int NB = outer_block<T>(n, split != nullptr, batch.count == 1);
     const int np = (n + NB - 1) / NB;
     hipStream_t main = h->stream, side = h->side, look = h->look;
     auto col = [&](int q) { return std::min(n, q * NB); };  // first column of panel q (n past the end)

@@ -240,6 +240,23 @@ def test_device_normals_match_the_oracle(handle):
         assert np.abs(got - want).max() <= 1e-14 * max(1.0, np.abs(want).max())
 
 
+def profiled_pposv(handle, a, b):
+    """(factor, solution, {class: (launches, ms, flops, bytes)}) of one profiled pposv."""
+    A = dd.DistributedMatrix.from_global_matrix(handle, a, mb=512, nb=512)
+    B = dd.DistributedMatrix.from_global_matrix(handle, b, mb=512, nb=512)
+    handle.profile(True)
+    try:
+        _, info = dd.pposv(A, B, "L")
+        prof = handle.profile_read()
+    finally:
+        handle.profile(False)
+    assert info == 0
+    for k, (cnt, ms, fl, _) in prof.items():
+        if cnt:
+            assert ms > 0, k
+    return A.to_global_matrix(), B.to_global_matrix(), prof
+
+
 def test_launch_profiler_records_the_schedule(handle):
     """The per-launch event profiler behind the benchmark's roofline figures:
     one FP64 pposv at n = 2048 (four 512-column panels, uplo L) records the
@@ -253,19 +270,28 @@ def test_launch_profiler_records_the_schedule(handle):
     n, nrhs = 2048, 4
     a = orc.spd_matrix(n, seed=14, delta=0.3)
     b = orc.normal_matrix(14, 1, n, nrhs)
-    A = dd.DistributedMatrix.from_global_matrix(handle, a, mb=512, nb=512)
-    B = dd.DistributedMatrix.from_global_matrix(handle, b, mb=512, nb=512)
-    handle.profile(True)
+    previous = dd.lib.ddla_c_set_panel_width(512)
     try:
-        _, info = dd.pposv(A, B, "L")
-        prof = handle.profile_read()
+        _, _, prof = profiled_pposv(handle, a, b)
     finally:
-        handle.profile(False)
-    assert info == 0
+        dd.lib.ddla_c_set_panel_width(previous)
     counts = {k: v[0] for k, v in prof.items()}
     assert counts["panel"] == 4 and counts["trailing_update"] == 1 and counts["lookahead_update"] == 5
     assert counts["solve"] == 1 and counts["trtri"] == 1
-    for k, (cnt, ms, fl, _) in prof.items():
-        if cnt:
-            assert ms > 0, k
     assert prof["trailing_update"][2] == 512 * 513 * 512
+
+
+def test_launch_profiler_leaves_the_call_as_it_is(handle):
+    """With the profiler on, the same launches run as without: one panel at n = 2048, and the same bits."""
+    from oracle import oracle as orc
+
+    n, nrhs = 2048, 4
+    a = orc.spd_matrix(n, seed=14, delta=0.3)
+    b = orc.normal_matrix(14, 1, n, nrhs)
+    factor, x, prof = profiled_pposv(handle, a, b)
+    counts = {k: v[0] for k, v in prof.items() if v[0]}
+    assert counts == {"panel": 1, "solve": 1, "trtri": 1}, counts
+    A = dd.DistributedMatrix.from_global_matrix(handle, a, mb=512, nb=512)
+    B = dd.DistributedMatrix.from_global_matrix(handle, b, mb=512, nb=512)
+    assert dd.pposv(A, B, "L")[1] == 0
+    assert A.to_global_matrix().tobytes() == factor.tobytes() and B.to_global_matrix().tobytes() == x.tobytes()
