@@ -359,7 +359,8 @@ int ddla_z_gemm_vbatched2s_mixed(void* handle, int real_operand, int ab1_real, c
  * logdet NaN) or -1 (invalid order / leading dimension).  Arrays are device
  * resident; asynchronous on the handle's stream.  _run allocates and
  * synchronizes nothing (graph-capturable); _tune times the schedules on
- * copies of the inputs and keeps the fastest in the handle; _graph captures
+ * copies of the inputs and keeps the fastest in the handle (in FP32, of those
+ * within 4 % of it, a left-looking one, which rounds less); _graph captures
  * one call into a replayable hipGraph owning its workspace.  Schedules: the
  * persistent fused kernel for every member, or -- for the members of more
  * than split_blocks 64-row blocks -- a blocked factorization whose trailing

@@ -110,12 +110,30 @@ void pposvVbatched(const DdlaHandle_t& h, char uplo, const int* d_n, T* const* d
                                          work, bytes);
 }
 
+// The tuner's choice among the timed schedules: the fastest one.  In FP32 a
+// left-looking schedule counts as tied with it up to 4 %, and is then taken: the
+// shorter of two timings of one schedule differs by up to 3.3 % from the next two
+// (batches of 500 to 4096 members), and the left-looking kernel rounds each element
+// of the trailing matrix once per block column instead of once per update.  1500
+// FP32 systems of orders 20 to 300: left-looking 506 to 518 us, log-determinants
+// 6.8e-8 off, solutions 2.7e-7; the fused right-looking schedule 496 to 512 us,
+// 9.6e-8, 3.9e-7.  In FP64 the difference is below 1e-16.
+std::size_t pick_batched_schedule(const std::vector<ScheduleTime>& times, std::size_t elem)
+{
+    const float tie = elem == sizeof(float) ? 0.96f : 1.0f;
+    auto cost = [&](const ScheduleTime& t) { return t.left_looking ? tie * t.ms : t.ms; };
+    const auto best = std::min_element(times.begin(), times.end(), [&](const ScheduleTime& a, const ScheduleTime& b) {
+        return cost(a) < cost(b);
+    });
+    return (std::size_t)(best - times.begin());
+}
+
 // Times every schedule (kernel variant for 1 or 2 workgroups per CU, largest
 // first or index order, and -- largest first only -- the blocked path for the
 // members of more than 2, 3, 4 or 6 blocks in steps of one or two block
 // columns, or the left-looking kernel for every member) on copies of the caller's
-// matrices, so the inputs are left unchanged, and keeps the fastest in the
-// handle for later calls.
+// matrices, so the inputs are left unchanged, and keeps the fastest
+// (pick_batched_schedule) in the handle for later calls.
 template <class T>
 void pposvVbatchedTune(const DdlaHandle_t& h, char uplo, const int* d_n, T* const* d_A, const int* d_lda, int nrhs,
                        T* const* d_B, const int* d_ldb, int batch, int max_n, int* occupancy, bool* ordered)
@@ -229,15 +247,9 @@ void pposvVbatchedTune(const DdlaHandle_t& h, char uplo, const int* d_n, T* cons
     DDLA_HIP(hipEventDestroy(e0));
     DDLA_HIP(hipEventDestroy(e1));
     DDLA_HIP(hipFree(base));
-    // The left-looking kernel rounds each element of the trailing matrix once
-    // per block column instead of once per update: on 1500 FP32 systems of
-    // orders 20 to 300 its log-determinants are 7.4e-8 off against 1.3e-7, its
-    // solutions 2.8e-7 against 4.6e-7.  So another schedule has to be faster by
-    // more than two timings of one schedule differ to be taken before it.
-    constexpr float kLeftLookingShare = 0.9f;
-    auto cost = [](const Candidate& c) { return c.left_looking ? kLeftLookingShare * c.ms : c.ms; };
-    const auto best = std::min_element(cands.begin(), cands.end(),
-                                       [&](const Candidate& a, const Candidate& b) { return cost(a) < cost(b); });
+    std::vector<ScheduleTime> times;
+    for (const Candidate& c : cands) times.push_back({c.ms, c.left_looking});
+    const Candidate* const best = &cands[pick_batched_schedule(times, sizeof(T))];
     tuning = DdlaStream::BatchedTuning{true,          best->occupancy,    best->ordered,
                                        best->split_blocks, best->left_looking, best->step_blocks};
     if (occupancy) *occupancy = best->occupancy;

@@ -167,6 +167,14 @@ template <class R>
 void diag_logdet(const DdlaHandle_t& h, int n, const std::complex<R>* A, int lda, std::complex<R>& result);
 } // namespace complex_impl
 
+// The index of the schedule that pposvVbatchedTune keeps among the timed ones of
+// a batch of elements of `elem` bytes (batched.cpp).
+struct ScheduleTime {
+    float ms;
+    bool left_looking;
+};
+std::size_t pick_batched_schedule(const std::vector<ScheduleTime>& times, std::size_t elem);
+
 // pposv's backend bytes and its run (ia = ja = ib = jb = 1, arguments already
 // checked; cholesky.cpp).  wide: with the 128-row solve sweeps where pposv takes
 // them (1 KB of work per row in FP64), else with the 64-row ones (512 bytes).

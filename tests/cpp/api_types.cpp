@@ -11,7 +11,8 @@
 //     direction (both triangles, with and without the diagonal, padding rows
 //     and the other triangle untouched, a 3-byte element type), events, device
 //     queries, the rank <-> grid maps and the descriptor-level index maps
-//     (include/ddla/ddla_desc.h:143-191).
+//     (include/ddla/ddla_desc.h:143-191);
+//   * the batched tuner's choice among timed schedules.
 // "api_types cpu" runs the index checks only (no GPU); no argument runs both.
 // Prints one line per failure and exits non-zero if any.
 #include <ddla/ddla.h>
@@ -247,9 +248,24 @@ static void handle_helpers_on_gpu(ddla::DdlaHandle_t h)
     EXPECT(ddla::ddlaGetStream(h) == before);
 }
 
+static void batched_schedule_choice()
+{
+    using ddla::pick_batched_schedule;
+    const std::size_t f = sizeof(float), d = sizeof(double);
+    // the fastest, in either type
+    EXPECT(pick_batched_schedule({{2.0f, false}, {1.0f, false}, {1.5f, true}}, d) == 1);
+    EXPECT(pick_batched_schedule({{1.0f, true}, {1.1f, false}}, f) == 0);
+    EXPECT(pick_batched_schedule({{1.0f, false}, {1.05f, true}}, f) == 0);
+    EXPECT(pick_batched_schedule({{1.0f, false}, {1.01f, true}}, d) == 0);
+    // a left-looking one that two timings cannot tell from it, in FP32
+    EXPECT(pick_batched_schedule({{1.0f, false}, {1.03f, true}, {1.02f, false}}, f) == 1);
+    EXPECT(pick_batched_schedule({{1.03f, true}, {1.0f, false}, {1.01f, true}}, f) == 2);
+}
+
 int main(int argc, char** argv)
 {
     index_maps();
+    batched_schedule_choice();
     if (!(argc > 1 && std::strcmp(argv[1], "cpu") == 0)) vector_on_gpu();
     std::printf("%s: %d failure(s)\n", argc > 1 ? argv[1] : "all", failures);
     return failures == 0 ? 0 : 1;

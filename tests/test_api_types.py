@@ -11,7 +11,8 @@ tests/cpp/api_types.cpp (built next to the library by the csrc Makefile):
     direction against element-wise expectations (both triangles, with and
     without the diagonal, padding and the other triangle untouched, a 3-byte
     element), events, device queries, the rank <-> grid maps and the argument
-    rules.
+    rules;
+  * the batched tuner's choice among timed schedules.
 """
 import os
 import subprocess
