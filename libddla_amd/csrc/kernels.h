@@ -68,7 +68,8 @@ void vbatched_validate(hipStream_t s, int na, int nb, const int* m, const int* n
 
 // Panel factorization of the blocked Cholesky (one persistent launch per
 // panel), T real or std::complex.  panel_factor factors columns [k, k + kb) (kb
-// <= 4096, every earlier trailing update applied) of the lower triangle at A:
+// <= 4096; k and, except at the matrix's end, kb multiples of 64; every earlier
+// trailing update applied) of the lower triangle at A:
 // the diagonal blocks, their inverses and the rows below.  On a non-positive or
 // NaN pivot in global column p (0-based) it sets *info = p + 1, and
 // kInfoWaitLimit if one of its waits gave up (unless *info was set first); it

@@ -83,7 +83,8 @@ void panel_factor(hipStream_t s, int n, T* A, long long lda, int k, int kb, int*
     using E = typename PanelElement<T>::type;
     if (kb <= 0 || k < 0 || k + kb > n) return;
     if (kb > kMaxCols * kB) throw std::invalid_argument("panel_factor: panel wider than 4096 columns");
-    if (k % kB != 0) throw std::invalid_argument("panel_factor: panel must start on a 64-column boundary");
+    if (k % kB != 0 || (kb % kB != 0 && k + kb < n))
+        throw std::invalid_argument("panel_factor: panel must start and, before the last column, end on a 64-column boundary");
     if (batch.count <= 0) return;
     PanelArgs<E> a{reinterpret_cast<E*>(A), lda, n, k, kb, info, static_cast<E*>(work),
                    panel_sync<T>(n, work) + (size_t)(k / kB) * sync_ints((int)panel_blocks(n)),

@@ -12,13 +12,15 @@
 //     and the other triangle untouched, a 3-byte element type), events, device
 //     queries, the rank <-> grid maps and the descriptor-level index maps
 //     (include/ddla/ddla_desc.h:143-191);
-//   * the batched tuner's choice among timed schedules.
+//   * the batched tuner's choice among timed schedules;
+//   * panels that the factorization's units cannot hold are refused.
 // "api_types cpu" runs the index checks only (no GPU); no argument runs both.
 // Prints one line per failure and exits non-zero if any.
 #include <ddla/ddla.h>
 #include <ddla/ddla_vector.h>
 
 #include "internal.h"  // white-box: the handle's own look-ahead streams
+#include "kernels.h"
 
 #include <cstdio>
 #include <cstring>
@@ -262,10 +264,28 @@ static void batched_schedule_choice()
     EXPECT(pick_batched_schedule({{1.03f, true}, {1.0f, false}, {1.01f, true}}, f) == 2);
 }
 
+// Refused on the host: the arguments are never used.
+static void panel_arguments()
+{
+    auto refused = [](int n, int k, int kb) {
+        try {
+            ddla::kern::panel_factor<double>(nullptr, n, nullptr, n, k, kb, nullptr, nullptr);
+        } catch (const std::invalid_argument&) {
+            return true;
+        }
+        return false;
+    };
+    EXPECT(refused(1000, 32, 64));     // starts inside a block
+    EXPECT(refused(1000, 0, 100));     // ends inside a block with rows below
+    EXPECT(refused(1000, 64, 935));
+    EXPECT(refused(9000, 0, 4160));    // wider than 64 block columns
+}
+
 int main(int argc, char** argv)
 {
     index_maps();
     batched_schedule_choice();
+    panel_arguments();
     if (!(argc > 1 && std::strcmp(argv[1], "cpu") == 0)) vector_on_gpu();
     std::printf("%s: %d failure(s)\n", argc > 1 ? argv[1] : "all", failures);
     return failures == 0 ? 0 : 1;

@@ -12,7 +12,8 @@ tests/cpp/api_types.cpp (built next to the library by the csrc Makefile):
     without the diagonal, padding and the other triangle untouched, a 3-byte
     element), events, device queries, the rank <-> grid maps and the argument
     rules;
-  * the batched tuner's choice among timed schedules.
+  * the batched tuner's choice among timed schedules, and the panels that the
+    factorization refuses.
 """
 import os
 import subprocess
