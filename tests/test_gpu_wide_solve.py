@@ -1,20 +1,20 @@
-"""The staged triangular solve (512-row stages) that ppotrs / pposv take from
-order 8192 with fewer than 256 right-hand sides.
+"""The solves over 128-row blocks at large orders with fewer than 256
+right-hand sides.
 
-Its arithmetic differs from the 64-row sweeps (explicit inverses of the
-512 x 512 diagonal blocks), so it is pinned against them and against the
+Their arithmetic differs from the 64-row sweeps (explicit inverses of the 128 x
+128 diagonal blocks, other sums), so they are pinned against them and against the
 problem itself:
-* FP64: the factor is the same computation (bit for bit equal to
-  ddla_d_pposv_noalloc's, which always takes the 64-row sweeps), and the
-  solutions agree within 1e-11 relative (kappa about 40); the normwise
-  backward error ||A X - B||_inf / (||A||_inf ||X||_inf) meets config 1's bar
-  0.05 n eps.  Orders on and off the stage grid (8192, 8200: a last stage of 8
-  rows, 9000), one and two right-hand-side slabs (70 columns), both triangles
-  and both sides.
+* FP64: the solution agrees with the one that two triangular solves (ptrtrs,
+  always the 64-row sweeps at these sizes) give with the same factor within
+  1e-11 relative (kappa about 40); ddla_d_pposv_noalloc, the same kernels on
+  the static scratch, gives the same bits; the normwise backward error ||A X -
+  B||_inf / (||A||_inf ||X||_inf) is within 0.05 n eps.  Orders on
+  and off the grid of blocks (8192, 8200: a last block of 8 rows, 9000), several
+  slabs of columns (70), both triangles and both sides.
 * FP32: backward error against the FP32 system within 0.05 n eps32.
-* The mixed-precision solver's corrections through the staged solve.
-* The wait limit forced from the host: the staged sweeps give up, every
-  workgroup exits, and the call reports the wait error.
+* The mixed-precision solver's corrections.
+* The wait limit forced from the host: the sweeps give up, every workgroup
+  exits, and the call reports the wait error.
 
 A and B are generated on the GPU (ddla_d_spd_generate / ddla_c_fill_normal).
 """
@@ -60,10 +60,10 @@ def backward_error(a, x, b, side):
 
 @pytest.mark.parametrize("n,nrhs,uplo,side", [(8192, 64, "L", "L"), (8200, 70, "U", "L"), (9000, 1, "L", "L"),
                                               (8200, 3, "U", "R")])
-def test_fp64_staged_matches_64_row_sweeps(handle, n, nrhs, uplo, side):
+def test_fp64_matches_64_row_sweeps(handle, n, nrhs, uplo, side):
     import torch
 
-    print(f"case staged FP64 n={n} nrhs={nrhs} uplo={uplo} side={side}", flush=True)
+    print(f"case wide solve FP64 n={n} nrhs={nrhs} uplo={uplo} side={side}", flush=True)
     rows, cols = (n, nrhs) if side == "L" else (nrhs, n)
     a0, b0 = generate(handle, n, 31, 0.1, rows, cols)
     out = []
@@ -79,19 +79,28 @@ def test_fp64_staged_matches_64_row_sweeps(handle, n, nrhs, uplo, side):
         assert info.value == 0
         out.append((a, b))
     (fa, xa), (fb, xb) = out
-    assert torch.equal(fa, fb)
-    rel = ((xa - xb).abs().max() / xb.abs().max()).item()
+    assert torch.equal(fa, fb) and torch.equal(xa, xb)
+    # A = L L^T or U^T U: X = A^-1 B (side L) or B A^-1 (side R) by two triangular solves
+    F = dd.DistributedMatrix.from_torch(handle, fa, n, n, 512, 512)
+    xs = b0.clone()
+    torch.cuda.synchronize()
+    X = dd.DistributedMatrix.from_torch(handle, xs, rows, cols, 512, 512)
+    for trans in ("NT" if (uplo == "L") == (side == "L") else "TN"):
+        dd.ptrtrs(F, X, side, uplo, trans)
+    handle.synchronize()
+    rel = ((xa - xs).abs().max() / xs.abs().max()).item()
     berr = backward_error(a0, xa, b0, side)
-    print(f"  staged vs 64-row sweeps {rel:.2e}, backward error {berr:.2e}", flush=True)
+    print(f"  128-row vs 64-row sweeps {rel:.2e}, backward error {berr:.2e}", flush=True)
+    assert not torch.equal(xa, xs)  # other sums: the routes are two
     assert rel <= 1e-11, rel
     assert berr <= 0.05 * n * EPS, berr
 
 
-def test_fp32_staged_backward_error(handle):
+def test_fp32_backward_error(handle):
     import torch
 
     n, nrhs = 8200, 70
-    print(f"case staged FP32 n={n} nrhs={nrhs}", flush=True)
+    print(f"case wide solve FP32 n={n} nrhs={nrhs}", flush=True)
     a0, b0 = generate(handle, n, 32, 0.1, n, nrhs)
     a32, b32 = a0.float(), b0.float()
     a, b = a32.clone(), b32.clone()
@@ -106,11 +115,11 @@ def test_fp32_staged_backward_error(handle):
 
 
 @pytest.mark.parametrize("factor", [dd.FACTOR_FP32, dd.FACTOR_BF16X3, dd.FACTOR_FP16X3])
-def test_mixed_refinement_through_staged_solve(handle, factor):
+def test_mixed_refinement(handle, factor):
     import torch
 
     n, nrhs, tol = 8200, 70, 1e-14
-    print(f"case staged mixed n={n} nrhs={nrhs} factor={factor}", flush=True)
+    print(f"case wide solve mixed n={n} nrhs={nrhs} factor={factor}", flush=True)
     a0, b0 = generate(handle, n, 33, 4e-4, n, nrhs)
     a, b = a0.clone(), b0.clone()
     A = dd.DistributedMatrix.from_torch(handle, a, n, n, 512, 512)
@@ -124,11 +133,11 @@ def test_mixed_refinement_through_staged_solve(handle, factor):
     assert berr <= tol
 
 
-def test_staged_wait_limit_reported(handle):
+def test_wait_limit_reported(handle):
     import torch
 
     n, nrhs = 8192, 8
-    print("case staged forced wait limit", flush=True)
+    print("case wide solve forced wait limit", flush=True)
     a0, b0 = generate(handle, n, 34, 0.5, n, nrhs)
     a = a0.clone()
     A = dd.DistributedMatrix.from_torch(handle, a, n, n, 512, 512)

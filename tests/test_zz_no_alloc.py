@@ -4,7 +4,8 @@ It runs the kernels of ddla_d_pposv on a static array instead of the handle's
 scratch, so its factor and solution must equal ddla_d_pposv's bit for bit on
 the same inputs.  Two calls in a row, the second smaller (the array keeps the
 first call's contents), both triangles and both sides; a failed pivot; the
-size limit; n = 0.  Each result is also checked against the oracle.
+size limit; n = 0; an order whose 128-row solve does not fit and whose 64-row one
+does.  Each result is also checked against the oracle or the problem itself.
 """
 import ctypes
 
@@ -63,6 +64,41 @@ def test_two_calls_match_pposv(handle, side, uplo):
         ref, rinfo = orc.potrf(uplo, a)
         assert rinfo == 0
         assert np.linalg.norm(tri(fa) - tri(ref)) <= 1e-12 * np.linalg.norm(tri(ref))
+
+
+def test_64_row_sweeps_where_the_128_row_ones_do_not_fit(handle):
+    """Side 'R' stages B^T in the scratch: n (8 nrhs + 1024) > 64 MiB > n (8 nrhs + 512).  pposv takes the
+    128-row sweeps there, with the same factor; the solutions agree within 1e-11 (kappa about 40)."""
+    import torch
+
+    n, nrhs = 24000, 255
+    assert n * (8 * nrhs + 1024) > 64 << 20 > n * (8 * nrhs + 512) + (1 << 20)
+    print(f"case pposv_noalloc 64-row sweeps n={n} nrhs={nrhs}", flush=True)
+    a0 = torch.empty((n, n), dtype=torch.float64, device="cuda")
+    work = torch.empty_like(a0)
+    b0 = torch.empty((n, nrhs), dtype=torch.float64, device="cuda")  # B is nrhs x n, column-major
+    torch.cuda.synchronize()
+    dd.check_status(dd.lib.ddla_d_spd_generate(handle.ptr, n, 45, 0.1, ctypes.c_void_p(a0.data_ptr()), n,
+                                               ctypes.c_void_p(work.data_ptr())))
+    dd.check_status(dd.lib.ddla_c_fill_normal(handle.ptr, 45, 1, 0, n * nrhs, ctypes.c_void_p(b0.data_ptr())))
+    handle.synchronize()
+    out = []
+    for entry, storage in ((dd.lib.ddla_d_pposv_noalloc, work), (dd.lib.ddla_d_pposv, torch.empty_like(a0))):
+        storage.copy_(a0)
+        b = b0.clone()
+        torch.cuda.synchronize()
+        A = dd.DistributedMatrix.from_torch(handle, storage, n, n, 512, 512)
+        B = dd.DistributedMatrix.from_torch(handle, b, nrhs, n, 512, 512)
+        st, info = call(entry, handle, "R", "L", n, nrhs, A, B)
+        assert st == 0 and info == 0, dd.lib.ddla_c_error_string(st)
+        out.append((storage, b))
+    (fa, xa), (fb, xb) = out
+    assert torch.equal(fa.tril(), fb.tril()) and torch.equal(fa.triu(), fb.triu())
+    assert not torch.equal(xa, xb)  # two routes
+    assert ((xa - xb).abs().max() / xb.abs().max()).item() <= 1e-11
+    # X A = B: row j of X in column j of xa
+    r = (b0 - torch.mm(a0, xa)).abs().amax(0) / (a0.abs().sum(1).max() * xa.abs().amax(0))
+    assert r.max().item() < 0.05 * n * EPS
 
 
 def test_failed_pivot_leaves_b(handle):
