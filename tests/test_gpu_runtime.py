@@ -154,6 +154,49 @@ def test_wait_limit_error_is_reported_and_handle_recovers(handle):
     assert orc.backward_error(a, x, b) < 1e-14
 
 
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+def test_complex_wait_limit_error_is_reported(handle, dtype):
+    """The same with the complex panels and sweeps (order 2048, 32 blocks)."""
+    import torch
+
+    n, nrhs = 2048, 5
+    tdtype = torch.complex128 if dtype is np.complex128 else torch.complex64
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    g = torch.randn(n, n, dtype=torch.complex128, device="cuda", generator=gen)
+    a = torch.mm(g, g.mH.contiguous()) / n
+    a = (0.5 * (a + a.mH)).contiguous()
+    a.diagonal().add_(0.5)
+    b0 = torch.randn(nrhs, n, dtype=torch.complex128, device="cuda", generator=gen)
+
+    def storage(x):
+        s = x.to(tdtype).clone(memory_format=torch.contiguous_format)
+        torch.cuda.synchronize()
+        return s
+
+    f = storage(a.t())
+    A = dd.DistributedMatrix.from_torch(handle, f, n, n)
+    assert dd.ppotrf(A, "L")[1] == 0
+    b, f2 = storage(b0), storage(a.t())
+    previous = dd.lib.ddla_c_set_wait_limit(1)
+    try:
+        assert previous == 1 << 23
+        print(f"case forced wait limit: {np.dtype(dtype).name} ppotrs", flush=True)
+        with pytest.raises(RuntimeError, match="wait limit"):
+            dd.ppotrs(A, dd.DistributedMatrix.from_torch(handle, b, n, nrhs), "L")
+        print(f"case forced wait limit: {np.dtype(dtype).name} ppotrf", flush=True)
+        with pytest.raises(RuntimeError, match="wait exceeded its limit"):
+            dd.ppotrf(dd.DistributedMatrix.from_torch(handle, f2, n, n), "L")
+    finally:
+        assert dd.lib.ddla_c_set_wait_limit(0) == 1
+    b, f2 = storage(b0), storage(a.t())
+    _, info = dd.pposv(dd.DistributedMatrix.from_torch(handle, f2, n, n),
+                       dd.DistributedMatrix.from_torch(handle, b, n, nrhs), "L")
+    assert info == 0
+    aw, x, rhs = a.to(tdtype).to(torch.complex128), b.t().to(torch.complex128).contiguous(), b0.to(tdtype).t()
+    r = (rhs.to(torch.complex128) - torch.mm(aw, x)).abs().amax(0) / (aw.abs().sum(1).max() * x.abs().amax(0))
+    assert r.max().item() <= 0.05 * n * np.finfo(dtype).eps
+
+
 def test_ppotrs_three_phase_matches_driver(handle):
     """ppotrs_workspace_size + ppotrs_run on caller scratch give the driver's
     result bit for bit; a workspace below the query is rejected."""
