@@ -74,7 +74,7 @@ int ddla_c_set_wait_limit(int spins);
 /* Panel width of the blocked factorization (the depth of its trailing
  * updates); no counterpart in the reference (its vendor potrf picks its own
  * blocking).  Process-wide: cols <= 0 restores the built-in rule (one panel up
- * to order 4096, 768 columns for FP64 from 16384, else 512); other values are rounded down to a
+ * to order 4096, complex128 3840; 768 columns for FP64 from 16384, else 512); other values are rounded down to a
  * multiple of 64 within [64, 768] (the bf16 split-product factorization caps
  * it at 512).  Returns the previous override (0 = none).  The factor does not
  * depend on it beyond rounding; it exists so that tests can run the wide
@@ -485,7 +485,7 @@ int ddla_c_spd_generate_batch(void* handle, int batch, const int* n, unsigned lo
  * factorization, 2 triangular-solve sweeps, 3 diagonal-block inverses, 4
  * refinement residual, 5 other, 6 look-ahead updates of the next two panels'
  * columns.  The launches are those that the call makes with the profiler off:
- * a factorization up to order 4096 is one launch of class 1. */
+ * a factorization up to order 4096 (complex128 3840) is one launch of class 1. */
 int ddla_c_profile(void* handle, int enable);
 int ddla_c_profile_read(void* handle, int cls, int* count, double* ms, double* flops, double* bytes);
 

@@ -39,24 +39,31 @@ constexpr int kIB = 64;  // diagonal block of potf2 and of the solves
 // * A single problem of order <= 4096 is one panel: its 64 x 64 blocks are units
 //   of one launch, whose chain of diagonal blocks (18 us each in FP64) is all
 //   that is left; by 512-column panels the chain also waits for the rows below
-//   each panel, the look-ahead update of the next and two stream hand-overs:
-//   n = 2048 took 1.0 ms then, 0.6 ms now.
+//   each panel, the look-ahead update of the next and two stream hand-overs.
+//   ppotrf as one panel / by 512 columns, us: FP64 n = 600: 223 / 285, 2000: 601 /
+//   786, 4096: 1295 / 1770; FP32 194 / 255, 479 / 656, 985 / 1349; complex64 302 /
+//   396, 910 / 1163, 2188 / 2831; complex128 455 / 569, 1361 / 1766, but n = 3840:
+//   3930 / 3977, 3968: 4372 / 4231, 4096: 4426 / 4358 (one unit a CU: the
+//   updates outlast the chain).  4096 is what a unit's flags allow.
 // * Beyond, deeper updates amortize each tile's C read-modify-write better, wider
-//   panels lengthen the panel chain: FP64 at n = 32768 ran 209.3 / 205.0 / 206.4
-//   ms with 512 / 768 / 1024, while at n = 8192 512 is best.
+//   panels lengthen the panel chain: FP64 ppotrf with 512 / 768, ms: n = 8192:
+//   5.52 / 5.49, 16384: 28.2 / 27.4, 32768: 190.6 / 186.7.  (1024 at 32768 took 0.7 %
+//   more than 768 with panels of one workgroup a block row.)  FP32 has kept 512: 3.84 /
+//   3.69, 15.6 / 15.1, 98.8 / 96.3 say that 768 would be the faster there too.
 // * A batch of problems fills the chip with 512-column panels, which leave more
 //   of the work to the trailing updates; the split-product path keeps 512 (its
 //   panel buffers hold 512 columns).
 // A process-wide override (set_panel_width; 0 = the rule above) lets tests
 // run narrower and the 768-column panels at small orders.
 std::atomic<int> g_panel_width{0};
-constexpr int kOnePanelOrder = 4096;
+template <class T>
+constexpr int kOnePanelOrder = sizeof(T) == 16 ? 3840 : 4096;
 template <class T>
 int outer_block(int n, bool split, bool one_panel = true)
 {
     const int w = g_panel_width.load(std::memory_order_relaxed);
     if (w > 0) return split ? std::min(w, 512) : w;
-    if (!split && one_panel && n <= kOnePanelOrder) return kOnePanelOrder;
+    if (!split && one_panel && n <= kOnePanelOrder<T>) return kOnePanelOrder<T>;
     return std::is_same<T, double>::value && n >= 16384 ? 768 : 512;
 }
 
@@ -246,7 +253,6 @@ void potrf_blocked(DdlaStream* h, bool upper, int n, T* A, long long lda, int* i
     }
     const LView<T> v{A, lda};
     const int NB = outer_block<T>(n, split != nullptr, batch.count == 1);
-    const int np = (n + NB - 1) / NB;
     hipStream_t main = h->stream, side = h->side, look = h->look;
     auto col = [&](int q) { return std::min(n, q * NB); };  // first column of panel q (n past the end)
     // factors panel q and splits its rows below the diagonal block into buf[q % 3]
@@ -274,7 +280,6 @@ void potrf_blocked(DdlaStream* h, bool upper, int n, T* A, long long lda, int* i
             update_lower<T>(h, st, cls, v, M, N, kb, T(-1), c_lo, k, c_lo, k, T(1), c_lo, c_lo, true, info, flops,
                             batch);
     };
-    (void)np;
     const hipStream_t streams[3] = {main, side, look};
     const hipEvent_t events[3] = {h->ev_panel, h->ev_look, h->ev_rest};
     for (const sched::Step& st : sched::potrf_schedule(n, NB)) {

@@ -493,8 +493,8 @@ __global__ __launch_bounds__(256, panel_occupancy<T>()) void panel_kernel(PanelA
     // the roundings shrink with the Schur complement, and its scale rounds once in
     // 64 terms.  FP64 solutions with a smooth kernel matrix of order 4096 are off by
     // 3.1e-13 so, by 1.8e-12 if A is added to one long sum (an elementwise
-    // factorization: 8.8e-13); FP32 complex factors of order 4500 by 8.4e-8, by
-    // 2.7e-7 if every term rounds at the scale of A.  False: the panel was abandoned.
+    // factorization: 8.8e-13); complex64 factors of order 4500 by 5.0e-8, by more than
+    // 2e-7 if every term rounds at the scale of A.  False: the panel was abandoned.
     auto form_block = [&](int t, int c, bool diag) __attribute__((always_inline)) -> bool {
         const long long rt = row_of(t), rc = row_of(c);
         const int ht = rows_in(t), wc = min(kB, a.kb - kB * c);

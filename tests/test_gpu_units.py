@@ -1,5 +1,5 @@
 """Factorizations and solves at the edges of their blocks: orders around the
-64-row blocks and the largest one-panel order (4096), the same matrix by narrow
+64-row blocks and the largest one-panel orders (4096; complex128 3840), the same matrix by narrow
 panels, complex elements, and the 128-row solve sweeps over orders, right-hand
 sides, triangles and sides.
 
@@ -66,7 +66,7 @@ def bound(n, dtype):
 
 @pytest.mark.parametrize("dtype,n", [(np.float64, n) for n in (65, 128, 191, 1000, 4032, 4096, 4160)] +
                          [(np.float32, n) for n in (129, 1500, 4095, 4097)] +
-                         [(np.complex128, n) for n in (1, 63, 65, 200, 1025)] +
+                         [(np.complex128, n) for n in (1, 63, 65, 200, 1025, 3840, 3841)] +
                          [(np.complex64, n) for n in (64, 130, 1500, 4161)])
 @pytest.mark.parametrize("uplo", ["L", "U"])
 def test_factor_units(handle, dtype, n, uplo):
