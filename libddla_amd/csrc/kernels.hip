@@ -733,7 +733,7 @@ void batched_pposv(hipStream_t s, bool upper, int batch, int nrhs, const int* n,
     check_launch("batched_pposv");
     // blocked path for the members of more than split_blocks blocks (needs the sorted order)
     if (left_looking) {
-        solve_detail::zero_ints_kernel<<<1, 64, 0, s>>>(queue, 1);
+        zero_counters(s, queue, 1);
         check_launch("batched_pposv");
         BatchArgs<T> a{batch, nrhs, upper ? 1 : 0, max_blocks, n, A, lda, B, ldb, info, logdet, order, queue, xinv,
                        nullptr};
@@ -797,7 +797,7 @@ void batched_pposv(hipStream_t s, bool upper, int batch, int nrhs, const int* n,
         check_launch("batched_pposv");
         first = count;
     }
-    solve_detail::zero_ints_kernel<<<1, 64, 0, s>>>(queue, 1);
+    zero_counters(s, queue, 1);
     check_launch("batched_pposv");
     BatchArgs<T> a{batch, nrhs, upper ? 1 : 0, max_blocks, n, A, lda, B, ldb, info, logdet, order, queue, xinv, first};
     if (occupancy == 2) batched_pposv_kernel<T, 2><<<grid, kThreads, 0, s>>>(a);
@@ -841,11 +841,11 @@ void potrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long l
     if (slabs > 65535) throw std::invalid_argument("potrs: too many right-hand sides for one launch");
     SolveArgs<T> a{n, nrhs, nblk, L, ldl, upper ? 1 : 0, dinv, B, ldb, static_cast<int*>(work), error, wait_limit()};
     const dim3 grid((unsigned)nblk, (unsigned)slabs), block(kThreads);
-    zero_ints_kernel<<<1, 256, 0, s>>>(a.sync, 2 * slabs);
+    zero_counters(s, a.sync, 2 * slabs);
     check_launch("potrs");
     solve_sweep_kernel<T, false><<<grid, block, 0, s>>>(a);
     check_launch("potrs");
-    zero_ints_kernel<<<1, 256, 0, s>>>(a.sync, 2 * slabs);
+    zero_counters(s, a.sync, 2 * slabs);
     check_launch("potrs");
     solve_sweep_kernel<T, true><<<grid, block, 0, s>>>(a);
     check_launch("potrs");
@@ -906,7 +906,7 @@ void wide_sweeps(hipStream_t s, bool upper, int n, int nrhs, const T* L, long lo
     WideArgs<T> a{n, nrhs, blocks(n), ns, L, ldl, static_cast<const T*>(work), B, ldb, vec, sync, error,
                   wait_limit()};
     const unsigned grid = (unsigned)(a.nblk * ns);
-    zero_counters_kernel<<<1, 256, 0, s>>>(sync, 4 * ns);
+    zero_counters(s, sync, 4 * ns);
     check_launch("wide_sweeps");
     if (upper) wide_sweep_kernel<T, false, false><<<grid, kWThreads, 0, s>>>(a);
     else wide_sweep_kernel<T, false, true><<<grid, kWThreads, 0, s>>>(a);
@@ -927,7 +927,7 @@ void trsm_sweep(hipStream_t s, bool upper, bool backward, int n, int nrhs, const
     if (slabs > 65535) throw std::invalid_argument("trsm_sweep: too many right-hand sides for one launch");
     SolveArgs<T> a{n, nrhs, nblk, L, ldl, upper ? 1 : 0, dinv, B, ldb, static_cast<int*>(work), error, wait_limit()};
     const dim3 grid((unsigned)nblk, (unsigned)slabs), block(kThreads);
-    zero_ints_kernel<<<1, 256, 0, s>>>(a.sync, 2 * slabs);
+    zero_counters(s, a.sync, 2 * slabs);
     check_launch("trsm_sweep");
     if (backward) solve_sweep_kernel<T, true><<<grid, block, 0, s>>>(a);
     else solve_sweep_kernel<T, false><<<grid, block, 0, s>>>(a);

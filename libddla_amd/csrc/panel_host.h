@@ -59,10 +59,16 @@ int* panel_error_word(int n, void* work)
 }
 
 // p[0, count) := 0 for each problem y (problem y's words stride bytes after problem 0's)
-static __global__ void zero_ints_batched_kernel(int* p, int count, long long stride)
+static __global__ void zero_ints_kernel(int* p, int count, long long stride)
 {
     int* q = reinterpret_cast<int*>(reinterpret_cast<char*>(p) + blockIdx.y * stride);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) q[i] = 0;
+}
+
+// The counters of a launch that waits inside, or a work queue: p[0, count) := 0.
+inline void zero_counters(hipStream_t s, int* p, int count)
+{
+    zero_ints_kernel<<<1, 256, 0, s>>>(p, count, 0);
 }
 
 template <class T>
@@ -71,7 +77,7 @@ void panel_reset(hipStream_t s, int n, void* work, const Batch& batch)
     if (batch.count <= 0) return;
     const int count = (int)panel_counters(n) + 1;
     const dim3 grid((unsigned)((count + 255) / 256), (unsigned)batch.count);
-    zero_ints_batched_kernel<<<grid, 256, 0, s>>>(panel_sync<T>(n, work), count, batch.stride);
+    zero_ints_kernel<<<grid, 256, 0, s>>>(panel_sync<T>(n, work), count, batch.stride);
     panel_check("panel_reset");
 }
 

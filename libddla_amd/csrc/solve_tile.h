@@ -500,11 +500,6 @@ __global__ __launch_bounds__(kThreads) void symm_residual_kernel(SymmArgs<T> a)
         }
 }
 
-__global__ void zero_ints_kernel(int* p, int count)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) p[i] = 0;
-}
-
 } // namespace solve_detail
 } // namespace kern
 } // namespace ddla

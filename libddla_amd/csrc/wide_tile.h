@@ -154,11 +154,6 @@ __global__ __launch_bounds__(256) void wide_inverse_kernel(bool upper, int n, co
     }
 }
 
-__global__ void zero_counters_kernel(int* p, int count)
-{
-    for (int i = threadIdx.x; i < count; i += blockDim.x) p[i] = 0;
-}
-
 // Grid: nslab * nblk workgroups, slabs fastest, so that all slabs advance together.
 // DIRECT: Op(t, q)'s rows run along a stored column, else along a stored row
 // (BACKWARD == upper; with both in one kernel FP64's forward sweep spilled with a lower

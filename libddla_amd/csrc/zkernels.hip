@@ -57,8 +57,8 @@ __device__ __forceinline__ Cx<R> conj(Cx<R> a)
 }
 
 // ---------------------------------------------------------------------------
-// GEMM tile: BM x BN of C per 256-thread workgroup, four wavefronts (2 x 2) of
-// (BM / 2) x (BN / 2), slabs of 16 columns of op(A) and rows of op(B) in LDS by
+// GEMM tile: 64 x 64 of C per 256-thread workgroup, four wavefronts (2 x 2) of
+// 32 x 32, slabs of 16 columns of op(A) and rows of op(B) in LDS by
 // planes, the next slab's loads in flight while one is multiplied.
 // ---------------------------------------------------------------------------
 using gemm_detail::kPad;
@@ -88,30 +88,30 @@ struct ZProblem {
 };
 
 // LDS elements of a tile's slabs (op(A)'s planes, then op(B)'s).
-template <int BM, int BN, bool ACPX, bool BCPX>
+template <bool ACPX, bool BCPX>
 constexpr int zslab_elems()
 {
-    return kK * ((ACPX ? 2 : 1) * (BM + kPad) + (BCPX ? 2 : 1) * (BN + kPad));
+    return kK * (kT + kPad) * ((ACPX ? 2 : 1) + (BCPX ? 2 : 1));
 }
 
-// One operand's slabs: D consecutive indices (rows of op(A) or columns of
+// One operand's slabs: kT consecutive indices (rows of op(A) or columns of
 // op(B)) by kK of the inner dimension, for the tile at origin o of `extent`.
-// along: the stored contiguous dimension is the D one.  Loads of a slab that
+// along: the stored contiguous dimension is that of the indices.  Loads of a slab that
 // reaches beyond the operand are clamped and dropped.
-template <class R, bool CPX, int D>
+template <class R, bool CPX>
 struct ZOperand {
-    static constexpr int PER = D * kK / kTh, LD = D + kPad;
+    static constexpr int PER = kT * kK / kTh, LD = kT + kPad;
     using E = std::conditional_t<CPX, Cx<R>, R>;
     const E* P;
     long long ld;
     int o, extent, k;
     bool along, conjugate;
     E v[PER];
-    __device__ int index(int e) const { const int i = threadIdx.x + kTh * e; return along ? i % D : i / kK; }
-    __device__ int inner(int e) const { const int i = threadIdx.x + kTh * e; return along ? i / D : i % kK; }
+    __device__ int index(int e) const { const int i = threadIdx.x + kTh * e; return along ? i % kT : i / kK; }
+    __device__ int inner(int e) const { const int i = threadIdx.x + kTh * e; return along ? i / kT : i % kK; }
     __device__ void load(int k0)
     {
-        if (o + D <= extent && k0 + kK <= k) {
+        if (o + kT <= extent && k0 + kK <= k) {
             const E* base = P + (along ? o + k0 * ld : k0 + o * ld);
 #pragma unroll
             for (int e = 0; e < PER; ++e) v[e] = base[along ? index(e) + inner(e) * ld : inner(e) + index(e) * ld];
@@ -129,7 +129,7 @@ struct ZOperand {
     // distinct banks (gemm_detail::spread).  'T' 'N' products of complex128, batches of
     // 4000 of order 16: 131 -> 107 us, 16 of order 512: 496 -> 356 us, together with the
     // wavefronts that have no element of C and multiply nothing.
-    __device__ int place(int k) const { return along ? 0 : spread<R, D>(k); }
+    __device__ int place(int k) const { return along ? 0 : spread<R, kT>(k); }
     __device__ void store(R* S) const
     {
 #pragma unroll
@@ -145,18 +145,18 @@ struct ZOperand {
     }
 };
 
-template <class R, int BM, int BN, bool ACPX, bool BCPX>
+template <class R, bool ACPX, bool BCPX>
 __device__ void ztile(const ZProblem<R>& p, int ti, int tj, R* smem)
 {
     using Op = Mfma<R>;
-    constexpr int TM = BM / 32, TN = BN / 32;
-    const int m0 = ti * BM, n0 = tj * BN;
+    constexpr int TM = kT / 32, TN = kT / 32;
+    const int m0 = ti * kT, n0 = tj * kT;
     if (m0 >= p.m || n0 >= p.n) return;
-    if (p.tri == 1 && (long long)(m0 + BM - 1) + p.diag < n0) return;  // wholly above the written lower part
-    if (p.tri == 2 && (long long)m0 + p.diag > n0 + BN - 1) return;    // wholly below the written upper part
+    if (p.tri == 1 && (long long)(m0 + kT - 1) + p.diag < n0) return;  // wholly above the written lower part
+    if (p.tri == 2 && (long long)m0 + p.diag > n0 + kT - 1) return;    // wholly below the written upper part
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+    const int wm = (wave & 1) * (kT / 2), wn = (wave >> 1) * (kT / 2);
     const int pair = sizeof(R) == 8 ? 4 * (lk >> 1) : 0;
     const bool any = m0 + wm < p.m && n0 + wn < p.n;  // the wavefront has elements of C
     // D^T = op(B)^T op(A)^T: lane l % 16 of an accumulator runs along i, C's contiguous dimension
@@ -170,8 +170,8 @@ __device__ void ztile(const ZProblem<R>& p, int ti, int tj, R* smem)
 #pragma unroll
             for (int c = 0; c < 2; ++c) acc[x][y][c] = sum[x][y][c] = typename Op::acc_t{0, 0, 0, 0};
     if (p.k > 0 && (p.alpha.re != R(0) || p.alpha.im != R(0))) {
-        using OpA = ZOperand<R, ACPX, BM>;
-        using OpB = ZOperand<R, BCPX, BN>;
+        using OpA = ZOperand<R, ACPX>;
+        using OpB = ZOperand<R, BCPX>;
         OpA a{static_cast<const typename OpA::E*>(p.A), p.lda, m0, p.m, p.k, p.opa == 0, p.opa == 2, {}};
         OpB b{static_cast<const typename OpB::E*>(p.B), p.ldb, n0, p.n, p.k, p.opb != 0, p.opb == 2, {}};
         R* const As = smem;
@@ -260,14 +260,14 @@ __device__ void ztile(const ZProblem<R>& p, int ti, int tj, R* smem)
     }
 }
 
-template <class R, int BM, int BN, bool ACPX, bool BCPX>
+template <class R, bool ACPX, bool BCPX>
 __global__ __launch_bounds__(kTh, 2) void zgemm_kernel(ZProblem<R> p, TileOrder o, const int* abort)
 {
-    __shared__ R smem[zslab_elems<BM, BN, ACPX, BCPX>()];
+    __shared__ R smem[zslab_elems<ACPX, BCPX>()];
     if (abort != nullptr && *abort != 0) return;
     int ti, tj;
     if (!map_tile(o, blockIdx.x, ti, tj)) return;
-    ztile<R, BM, BN, ACPX, BCPX>(p, ti, tj, smem);
+    ztile<R, ACPX, BCPX>(p, ti, tj, smem);
 }
 
 template <class R>
@@ -283,7 +283,7 @@ struct ZBatch {
 template <class R, bool ACPX, bool BCPX>
 __global__ __launch_bounds__(kTh, 2) void zgemm_vbatched_kernel(ZBatch<R> v)
 {
-    __shared__ R smem[zslab_elems<kT, kT, ACPX, BCPX>()];
+    __shared__ R smem[zslab_elems<ACPX, BCPX>()];
     const int b = v.z0 + blockIdx.z;
     if (b >= v.batch) return;
     ZProblem<R> p;
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(kTh, 2) void zgemm_vbatched_kernel(ZBatch<R> v)
     p.ldc = v.ldc[b];
     p.tri = 0;
     p.diag = 0;
-    ztile<R, kT, kT, ACPX, BCPX>(p, blockIdx.x, blockIdx.y, smem);
+    ztile<R, ACPX, BCPX>(p, blockIdx.x, blockIdx.y, smem);
 }
 
 // inv(block b) = L(b, b)^-1 for every 64 x 64 diagonal block of a factor.
@@ -440,22 +440,22 @@ __global__ void zlogdet_final_kernel(const double* pmag, const double* pphase, c
     *reinterpret_cast<int*>(out + 2) = f;
 }
 
-template <class R, int BM, int BN>
+template <class R>
 void launch_zgemm(hipStream_t s, bool ac, bool bc, const ZProblem<R>& p, const int* abort)
 {
     TileOrder o;
-    o.ntm = (p.m + BM - 1) / BM;
-    o.ntn = (p.n + BN - 1) / BN;
-    o.lower_enum = (p.tri == 1 && p.diag == 0 && p.m == p.n && BM == BN) ? 1 : 0;
+    o.ntm = (p.m + kT - 1) / kT;
+    o.ntn = (p.n + kT - 1) / kT;
+    o.lower_enum = (p.tri == 1 && p.diag == 0 && p.m == p.n) ? 1 : 0;
     const long long total = o.lower_enum ? (long long)o.ntm * (o.ntm + 1) / 2 : (long long)o.ntm * o.ntn;
     if (total > (long long)INT_MAX / 2) throw std::invalid_argument("zgemm: problem too large for one launch");
     o.total = (int)total;
     o.group = 8;
     o.per_xcd = (o.total + 7) / 8;
     const unsigned grid = (unsigned)(o.per_xcd * 8);
-    if (ac && bc) zgemm_kernel<R, BM, BN, true, true><<<grid, kTh, 0, s>>>(p, o, abort);
-    else if (ac) zgemm_kernel<R, BM, BN, true, false><<<grid, kTh, 0, s>>>(p, o, abort);
-    else if (bc) zgemm_kernel<R, BM, BN, false, true><<<grid, kTh, 0, s>>>(p, o, abort);
+    if (ac && bc) zgemm_kernel<R, true, true><<<grid, kTh, 0, s>>>(p, o, abort);
+    else if (ac) zgemm_kernel<R, true, false><<<grid, kTh, 0, s>>>(p, o, abort);
+    else if (bc) zgemm_kernel<R, false, true><<<grid, kTh, 0, s>>>(p, o, abort);
     else throw std::invalid_argument("zgemm: at least one complex operand");
     zcheck_launch("zgemm");
 }
@@ -494,7 +494,7 @@ void zgemm(hipStream_t s, bool a_complex, bool b_complex, char ta, char tb, int 
     p.ldc = ldc;
     p.tri = tri;
     p.diag = diag;
-    launch_zgemm<R, kT, kT>(s, a_complex, b_complex, p, abort);
+    launch_zgemm<R>(s, a_complex, b_complex, p, abort);
 }
 
 template <class R>
@@ -570,7 +570,7 @@ void zpotrs_sweeps(hipStream_t s, bool upper, int n, int nrhs, const std::comple
     SweepArgs<R> a{n, nrhs, (n + kSB - 1) / kSB, reinterpret_cast<const Cx<R>*>(A), lda, upper ? 1 : 0,
                    reinterpret_cast<const Cx<R>*>(dinv), reinterpret_cast<Cx<R>*>(B), ldb, static_cast<int*>(sync),
                    error, wait_limit()};
-    zero_counters_kernel<<<1, 256, 0, s>>>(a.sync, 4 * ns);
+    zero_counters(s, a.sync, 4 * ns);
     const dim3 grid((unsigned)a.nblk, (unsigned)ns);
     sweep_kernel<R, false><<<grid, kSThreads, 0, s>>>(a);
     a.sync += 2 * ns;

@@ -57,11 +57,6 @@ struct SweepArgs {
     int spin_limit;
 };
 
-__global__ void zero_counters_kernel(int* p, int count)
-{
-    for (int i = threadIdx.x; i < count; i += blockDim.x) p[i] = 0;
-}
-
 template <class R, bool BACKWARD>
 __global__ __launch_bounds__(kSThreads) void sweep_kernel(SweepArgs<R> a)
 {
