@@ -630,7 +630,9 @@ def main():
     t = sum(times) / len(times)
     flops = n ** 3 / 3 + 2.0 * n ** 2 * nrhs
     value = flops / t / 1e12
-    cnt, ms, fl, _ = prof["trailing_update"]
+    # small orders are one panel, without trailing updates
+    phase = "trailing_update" if prof["trailing_update"][0] else "panel"
+    cnt, ms, fl, _ = prof[phase]
     achieved = fl / (ms / 1e3) / 1e12 if ms > 0 else 0.0
     breakdown = {k: {"launches": v[0] // max(1, args.steps), "ms_per_step": round(v[1] / args.steps, 3)}
                  for k, v in prof.items() if v[0]}
@@ -644,7 +646,7 @@ def main():
                        "bound": "the 128-row-block dependency chain (latency), not HBM"}
     traffic = None
     tfile = os.path.join(ROOT, "profiles", "trailing_update_traffic.json")
-    if os.path.exists(tfile):
+    if phase == "trailing_update" and os.path.exists(tfile):
         with open(tfile) as f:
             traffic = json.load(f).get("hbm_bytes_per_launch")
 
@@ -665,7 +667,9 @@ def main():
                    "nrhs": nrhs, "nb": 512, "panel_width": 768 if n >= 16384 else 512 if n > 4096 else n, "uplo": args.uplo},
         "pct_fp64_peak": round(100 * value / FP64_PEAK, 2),
         "backward_error": bwd,
-        "roofline": {"bound": "mfma", "kernel": "trailing_update (FP64 MFMA syrk)", "achieved": round(achieved, 3),
+        "roofline": {"bound": "mfma", "kernel": {"trailing_update": "trailing_update (FP64 MFMA syrk)",
+                                                "panel": "panel (the whole factorization)"}[phase],
+                     "achieved": round(achieved, 3),
                      "peak": FP64_PEAK, "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK, 4),
                      "traffic": traffic,
                      "traffic_source": "profiles/trailing_update_traffic.json (rocprofv3 FETCH_SIZE + WRITE_SIZE "

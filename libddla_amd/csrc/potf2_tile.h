@@ -18,7 +18,7 @@
 //     chain to the next one nor the strip has any exchange between wavefronts in
 //     it, and the pass turns the identity into L(b, b)^-T, the inverse of the
 //     strip's diagonal block (multiplied by an explicit inverse of the 4 x 4
-//     block instead, at the same speed, the columns of a nearly singular one were
+//     block instead, in 7.3 and 5.1 us a block, the columns of a nearly singular one were
 //     off by 47 n eps instead of 0.5, pivots among them down to negative ones in
 //     a factor reported complete, and a NaN pivot reached the columns before it);
 //   * between two passes the strip is applied to the next strip's columns
@@ -28,7 +28,7 @@
 //     L(r, k) X(k, c).
 // What bounds it is the dependency chain of 64 pivots; after the last strip
 // only one 16 x 16 product is left of the inverse.  Measured on one workgroup,
-// factor and inverse of a block: FP64 13.4 -> 7.3 us, FP32 9.6 -> 5.1 us against
+// factor and inverse of a block: FP64 13.4 -> 7.6 us, FP32 9.6 -> 5.4 us against
 // strips factored column by column in one wavefront (pivots and multipliers
 // through v_readlane) with the inverse formed afterwards.
 #pragma once
