@@ -60,8 +60,8 @@ def test_nearly_singular_blocks(handle, dtype):
     rng = np.random.RandomState(11)
     wide = np.clongdouble if np.dtype(dtype).kind == "c" else np.longdouble
     complete = 0
-    for trial in range(240):
-        n = rng.randint(2, 65)
+    for trial in range(600):
+        n = rng.randint(2, 20 if trial < 500 else 65)  # small ones: a pivot is tiny beside a large one more often
         a = nearly_singular(dtype, n, rng.randint(1, n + 1), rng.choice([0, 0.5, 1, 2, 8, 100, 1e4]), rng)
         A = dd.DistributedMatrix.from_global_matrix(handle, a)
         if dd.ppotrf(A, "L")[1] != 0:
@@ -72,7 +72,7 @@ def test_nearly_singular_blocks(handle, dtype):
         diag = np.sqrt(np.diagonal(a).real.astype(np.longdouble))
         off = np.abs(np.tril(a.astype(wide) - low @ low.conj().T)) / np.outer(diag, diag)
         assert off.max() <= 2 * (n + 3) * np.finfo(dtype).eps, (trial, n, float(off.max()))
-    assert complete >= 60
+    assert complete >= 200
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128, np.complex64])
